@@ -120,6 +120,10 @@ int prox_fl2d_num_waves(int W, int H, int nz, int n_tv, int row_chunk);
 int prox_fl2d_auto_rows(int W, int H, int nz, int n_tv);
 bool prox_fl2d_supported(int n_tv);
 hipError_t prox_fl2d(const ProxLaunch& a, hipStream_t s);
+// The same prox for iterates that are mostly non-zero: reads and writes every line and takes no
+// maps (prox_fl2d_num_waves partial rows, its own rule for the rows per wave).
+int prox_fl2d_dense_auto_rows(int W, int H, int nz, int n_tv);
+hipError_t prox_fl2d_dense(const ProxLaunch& a, hipStream_t s);
 
 int prox_l1_num_blocks(int W, int H, int nz);
 hipError_t prox_l1(const ProxLaunch& a, hipStream_t s);

@@ -29,15 +29,19 @@ namespace rihvr {
 
 constexpr int kDefaultRowChunk = 128;  // output rows per wave
 constexpr int kProxWaves = 4;    // waves per workgroup
+constexpr int kMinRowChunk = 4;  // fewest output rows per wave that a rule picks
 constexpr int kMaxNtv = 10;
 
 struct ProxGeom {
     int ow, nstrips, rc, nchunks;
 };
+// halo columns on each side of a wave's strip: one per TV iteration, and at least the left
+// neighbour of the objective's TV term
+constexpr int prox_halo(int n_tv) { return n_tv > 0 ? n_tv : 1; }
 inline ProxGeom prox_geom(int W, int H, int n, int row_chunk) {
     if (row_chunk <= 0) row_chunk = kDefaultRowChunk;
     ProxGeom g;
-    g.ow = 64 - 2 * n;
+    g.ow = 64 - 2 * prox_halo(n);
     if (g.ow > W) g.ow = W;
     g.nstrips = (W + g.ow - 1) / g.ow;
     g.rc = H < row_chunk ? H : row_chunk;
@@ -116,6 +120,7 @@ __device__ __forceinline__ float soft_fast(float v, float thr) {
 // slot and row parity is a compile-time constant and the ring is registers.
 template <int NTV> struct ProxWave {
     static constexpr int P = NTV + 3;
+    static constexpr int HX = prox_halo(NTV);
     static constexpr int U = (P % 2 == 0) ? P : 2 * P;
     float4 gd[2][NTV + 1];
     float2 yh[2][NTV + 1];
@@ -137,6 +142,7 @@ template <int NTV> struct ProxWave {
     uint64_t wlines = ~0ull, outlines = ~0ull;
     uint64_t plane_bits = 0;  // lines this wave set in the new map (its plane word's share)
     float acc_ls1 = 0.f, acc_ls2 = 0.f, acc_rs = 0.f, acc_l1 = 0.f, acc_tv = 0.f, acc_nnz = 0.f;
+    unsigned nnzy = 0;  // output voxels != 0 (wave-uniform)
     float smom = 0.f;  // the momentum step s of x0 = y0 + s (y0 - ym)
 
     static __device__ __forceinline__ int wrap_row(int tau, int H) {
@@ -290,15 +296,16 @@ template <int NTV> struct ProxWave {
             uint64_t m = 0ull;
             if (live) {
                 m = __builtin_amdgcn_ballot_w64(out_lane && (yv.x != 0.0f || yv.y != 0.0f));
+                nnzy += (unsigned)__popcll(m);
                 if (m) {
-                    // lanes NTV .. NTV + ow - 1 hold columns strip*ow + (lane - NTV): the lines
+                    // lanes HX .. HX + ow - 1 hold columns strip*ow + (lane - HX): the lines
                     // touched by non-zero lanes, then one atomic OR per row and wave
-                    const int c0 = strip * a.geo.ow - NTV;  // column of lane 0
+                    const int c0 = strip * a.geo.ow - HX;  // column of lane 0
                     uint64_t bits = 0;
-                    const int l_last = min(c0 + NTV + a.geo.ow - 1, W - 1) >> a.lsh;
-                    for (int l = (c0 + NTV) >> a.lsh; l <= l_last; ++l) {
-                        const int lo = max((l << a.lsh) - c0, NTV);
-                        const int hi = min((l << a.lsh) + (1 << a.lsh) - 1 - c0, NTV + a.geo.ow - 1);
+                    const int l_last = min(c0 + HX + a.geo.ow - 1, W - 1) >> a.lsh;
+                    for (int l = (c0 + HX) >> a.lsh; l <= l_last; ++l) {
+                        const int lo = max((l << a.lsh) - c0, HX);
+                        const int hi = min((l << a.lsh) + (1 << a.lsh) - 1 - c0, HX + a.geo.ow - 1);
                         if (lo > hi || lo > 63) continue;
                         const uint64_t lanes =
                             (hi >= 63 ? ~0ull : ((1ull << (hi + 1)) - 1ull)) & ~((1ull << lo) - 1ull);
@@ -406,9 +413,10 @@ __global__ void __launch_bounds__(64 * kProxWaves)
     const int chunk = rem / geo.nstrips;
     const int strip = rem - chunk * geo.nstrips;
     const int W = a.W;
-    const int ocol = strip * geo.ow + (lane - NTV);  // output column of this lane
-    const bool out_lane = (lane - NTV) >= 0 && (lane - NTV) < geo.ow && ocol < W;
-    const int xcol = wrapi(strip * geo.ow - NTV + lane, W);
+    constexpr int HX = prox_halo(NTV);
+    const int ocol = strip * geo.ow + (lane - HX);  // output column of this lane
+    const bool out_lane = (lane - HX) >= 0 && (lane - HX) < geo.ow && ocol < W;
+    const int xcol = wrapi(strip * geo.ow - HX + lane, W);
     const unsigned xoff = (unsigned)xcol * (unsigned)sizeof(float2);  // byte offset in a row
     const int r0 = chunk * geo.rc;
     const int r1 = min(a.H, r0 + geo.rc);
@@ -475,7 +483,231 @@ __global__ void __launch_bounds__(64 * kProxWaves)
         p[PS_L1X0] = s_l1;
         p[PS_TVX0] = s_tv;
         p[PS_NNZX0] = s_nnz;
-        p[PS_NNZY] = 0.0;
+        p[PS_NNZY] = (double)st.nnzy;
+        p[7] = 0.0;
+    }
+}
+
+// ----------------------------------------------------------------------------
+// The same prox for iterates that are mostly non-zero.  k_prox_fl2d earns its speed from the rows
+// it skips; where nearly every row holds data it runs at the latency of the loads it makes at
+// their own step (y_{k-1}, y_{k-2}, and the re-reads of a row that reduces): 435 us per call at
+// 512^2 x 100 with 47-99 % non-zeros, against about 220 us of VALU issue and 165 us of HBM time.
+// Here nothing is tested and everything is loaded ahead: a row's y_{k-1}, y_{k-2} and g two steps
+// before its x-hat is formed, and again (from the caches) one step before its output reduces; the
+// terms of x0 alone (L1, TV, non-zeros) are taken where x0 is formed.  No line map is read or
+// built: the output has none, so every line of it is read, which is what a dense volume needs.
+// 112 VGPRs, 4 waves per SIMD: 435 -> 270 us at 512^2 x 100, 98 -> 36 at 256^2 x 32, 72 -> 16 at
+// 64^2 x 8 (there with shorter row chunks too, see prox_fl2d_dense_auto_rows); it issues about
+// 85 % of the VALU's slots.  Two columns per lane (a halo of 12 in 128 instead of 10 in 64) need
+// 214 VGPRs and ran at 250-276 us and 44-49 us at the first two sizes: no better, not kept.
+// The arithmetic of every voxel is k_prox_fl2d's, so the volumes are the same bits; the sums add
+// the same terms in another order.
+// ----------------------------------------------------------------------------
+template <int NTV> struct DenseWave {
+    static constexpr int P = NTV + 3;
+    static constexpr int U = (P % 2 == 0) ? P : 2 * P;
+    float4 gd[2][NTV + 1];
+    float2 yh[2][NTV + 1];
+    float2 hist[P];                   // x-hat of the last rows, by compile-time slots
+    float2 py0[2], pym[2], pg[2];     // rows tau and tau + 1
+    float2 ry0, rym, rg;              // the row that is output next
+    float2 x0u;                       // x0 of the row above
+    float acc_ls1 = 0.f, acc_ls2 = 0.f, acc_rs = 0.f, acc_l1 = 0.f, acc_tv = 0.f, acc_nnz = 0.f;
+    unsigned nnzy = 0;                // wave-uniform
+    float smom = 0.f;
+    const char *y0p, *ymp, *gp;
+    char* yp;
+    unsigned rowb;
+    int row_ld;                       // row of the next load
+
+    static __device__ __forceinline__ float2 at(const char* base, unsigned off, unsigned xoff) {
+        return *(const float2*)(base + off + xoff);
+    }
+    __device__ __forceinline__ void load_row(int slot, int H, unsigned xoff) {
+        const unsigned off = (unsigned)row_ld * rowb;
+        py0[slot] = at(y0p, off, xoff);
+        pym[slot] = at(ymp, off, xoff);
+        pg[slot] = at(gp, off, xoff);
+        row_ld = row_ld + 1 == H ? 0 : row_ld + 1;
+    }
+    __device__ __forceinline__ float2 mom(float2 y0, float2 ym) const {
+        return make_float2(fmaf(smom, y0.x - ym.x, y0.x), fmaf(smom, y0.y - ym.y, y0.y));
+    }
+
+    template <int S>
+    __device__ __forceinline__ void step(const ProxDev& a, int tau, int r0, int r1, unsigned xoff, int ocol,
+                                         bool out_lane, int tau_end) {
+        constexpr int SLOT = S % P;
+        constexpr int PAR = S & 1;
+        constexpr int Q = PAR ^ 1;
+        // ---- row tau: x0, x-hat, and the objective terms of x0 ----
+        {
+            const float2 g = pg[PAR];
+            const float2 x0 = mom(py0[PAR], pym[PAR]);
+            hist[SLOT] = make_float2(fmaf(-a.t, g.x, x0.x), fmaf(-a.t, g.y, x0.y));
+            if (tau + 2 <= tau_end) load_row(PAR, a.H, xoff);
+            if (tau >= r0 && tau < r1) {
+                const float lr = lane_from_left(x0.x), li = lane_from_left(x0.y);
+                if (out_lane) {
+                    const float m2 = fmaf(x0.x, x0.x, x0.y * x0.y);
+                    acc_l1 += __builtin_amdgcn_sqrtf(m2);
+                    acc_nnz += (x0.x != 0.0f || x0.y != 0.0f) ? 1.0f : 0.0f;
+                    const float gxx = lr - x0.x, gyx = x0u.x - x0.x, gxy = li - x0.y, gyy = x0u.y - x0.y;
+                    acc_tv += __builtin_amdgcn_sqrtf(fmaf(gxx, gxx, fmaf(gxy, gxy, fmaf(gyx, gyx, gyy * gyy))));
+                }
+            }
+            x0u = x0;
+        }
+        // ---- TV levels: level k works on row tau - k ----
+#pragma unroll
+        for (int k = 1; k <= NTV; ++k) {
+            const float2 xh = hist[(SLOT - k + 2 * P) % P];
+            float2 y;
+            float4 go;  // g_{k-1} at row tau - k
+            if (k == 1) {
+                y = xh;
+                go = make_float4(0.f, 0.f, 0.f, 0.f);
+            } else {
+                go = gd[Q][k - 1];
+                const float4 gb = gd[PAR][k - 1];  // row below
+                const float dvr = lane_from_right(go.x) - go.x + gb.z - go.z;
+                const float dvi = lane_from_right(go.y) - go.y + gb.w - go.w;
+                y = make_float2(fmaf(-a.mu, dvr, xh.x), fmaf(-a.mu, dvi, xh.y));
+            }
+            const float2 yu = yh[Q][k];
+            const float axr = fmaf(a.sc, lane_from_left(y.x) - y.x, go.x);
+            const float axi = fmaf(a.sc, lane_from_left(y.y) - y.y, go.y);
+            const float ayr = fmaf(a.sc, yu.x - y.x, go.z);
+            const float ayi = fmaf(a.sc, yu.y - y.y, go.w);
+            // projection: by max(|a|, 1); a wave with no lane above 1 skips it (a factor of exactly 1)
+            gd[PAR][k] = make_float4(axr, axi, ayr, ayi);
+            const float n2 = fmaf(axr, axr, fmaf(axi, axi, fmaf(ayr, ayr, ayi * ayi)));
+            const bool proj = n2 > 1.0f;
+            if (__builtin_amdgcn_ballot_w64(proj)) {
+                const float inv = proj ? __builtin_amdgcn_rsqf(n2) : 1.0f;
+                gd[PAR][k] = make_float4(axr * inv, axi * inv, ayr * inv, ayi * inv);
+            }
+            yh[PAR][k] = y;
+        }
+        // ---- row o = tau - NTV - 1: estimate, threshold, output and reductions ----
+        const int o = tau - NTV - 1;
+        if (o >= r0 && o < r1) {
+            const float2 xh = hist[(SLOT - NTV - 1 + 2 * P) % P];
+            float2 yv;
+            if constexpr (NTV == 0) {
+                yv = xh;
+            } else {
+                const float4 gu = gd[Q][NTV];
+                const float4 gb = gd[PAR][NTV];
+                const float dvr = lane_from_right(gu.x) - gu.x + gb.z - gu.z;
+                const float dvi = lane_from_right(gu.y) - gu.y + gb.w - gu.w;
+                yv = make_float2(fmaf(-a.mu, dvr, xh.x), fmaf(-a.mu, dvi, xh.y));
+            }
+            if (a.do_soft) yv = make_float2(soft_fast(yv.x, a.thr), soft_fast(yv.y, a.thr));
+            yv = make_float2(yv.x + 0.0f, yv.y + 0.0f);  // zeros are +0
+            nnzy += (unsigned)__popcll(__builtin_amdgcn_ballot_w64(out_lane && (yv.x != 0.0f || yv.y != 0.0f)));
+            if (out_lane) {
+                *(float2*)(yp + (unsigned)o * rowb + xoff) = yv;
+                const float2 x0 = mom(ry0, rym);
+                const float dr = yv.x - x0.x, di = yv.y - x0.y;
+                acc_ls1 = fmaf(dr, rg.x, fmaf(di, rg.y, acc_ls1));
+                acc_ls2 = fmaf(dr, dr, fmaf(di, di, acc_ls2));
+                const float dre = (x0.x - yv.x) * (yv.x - ry0.x);
+                const float dim = (x0.y - yv.y) * (yv.y - ry0.y);
+                const int off = ((o * a.W) + ocol) & 1023;
+                acc_rs += off < 512 ? fmaf(2.0f, dim, dre) : dim;
+            }
+        }
+        // the next output row's y_{k-1}, y_{k-2} and g, read again one step ahead of their use
+        if (o + 1 >= r0 && o + 1 < r1) {
+            const unsigned on = (unsigned)(o + 1) * rowb;
+            ry0 = at(y0p, on, xoff);
+            rym = at(ymp, on, xoff);
+            rg = at(gp, on, xoff);
+        }
+    }
+
+    template <int... S>
+    __device__ __forceinline__ void block(std::integer_sequence<int, S...>, const ProxDev& a, int tau, int r0, int r1,
+                                          unsigned xoff, int ocol, bool out_lane, int tau_end) {
+        (step<S>(a, tau + S, r0, r1, xoff, ocol, out_lane, tau_end), ...);
+    }
+    template <int... S>
+    __device__ __forceinline__ void tail(std::integer_sequence<int, S...>, int rem, const ProxDev& a, int tau, int r0,
+                                         int r1, unsigned xoff, int ocol, bool out_lane, int tau_end) {
+        ((S < rem ? step<S>(a, tau + S, r0, r1, xoff, ocol, out_lane, tau_end) : void()), ...);
+    }
+};
+
+// waves per SIMD that the kernel's registers are held to (above 5 TV iterations: what they need)
+template <int NTV> constexpr int dense_waves_per_simd() { return NTV <= 5 ? 4 : 1; }
+
+template <int NTV>
+__global__ void __launch_bounds__(64 * kProxWaves)
+    __attribute__((amdgpu_waves_per_eu(dense_waves_per_simd<NTV>()))) k_prox_fl2d_dense(ProxDev a) {
+    using PW = DenseWave<NTV>;
+    constexpr int U = PW::U;
+    const int lane = threadIdx.x & 63;
+    const int wl = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // neighbouring strips, which read each other's halo columns, run on one XCD
+    const int w = xcd_local_block(blockIdx.x, gridDim.x) * kProxWaves + wl;
+    if (w >= a.nwaves) return;  // whole wave exits; no barriers below
+    const ProxGeom geo = a.geo;
+    const int per_plane = geo.nstrips * geo.nchunks;
+    const int z = w / per_plane;
+    const int rem = w - z * per_plane;
+    const int chunk = rem / geo.nstrips;
+    const int strip = rem - chunk * geo.nstrips;
+    constexpr int HX = prox_halo(NTV);
+    const int ocol = strip * geo.ow + (lane - HX);  // output column of this lane
+    const bool out_lane = (lane - HX) >= 0 && (lane - HX) < geo.ow && ocol < a.W;
+    const unsigned xoff = (unsigned)wrapi(ocol, a.W) * (unsigned)sizeof(float2);  // byte offset in a row
+    const int r0 = chunk * geo.rc;
+    const int r1 = min(a.H, r0 + geo.rc);
+    const size_t plane_off = (size_t)z * a.H * a.W;
+
+    PW st;
+    st.smom = a.s_mom_dev ? *a.s_mom_dev : a.s_mom;
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int k = 0; k <= NTV; ++k) {
+            st.gd[p][k] = make_float4(0.f, 0.f, 0.f, 0.f);
+            st.yh[p][k] = make_float2(0.f, 0.f);
+        }
+    st.x0u = st.ry0 = st.rym = st.rg = make_float2(0.f, 0.f);
+    const int tau0 = r0 - (NTV > 0 ? NTV : 1);
+    const int tau1 = r1 + NTV;  // inclusive
+    st.y0p = (const char*)(a.Y0 + plane_off);
+    st.ymp = (const char*)(a.YM + plane_off);
+    st.gp = (const char*)(a.G + plane_off);
+    st.yp = (char*)(a.Y + plane_off);
+    st.rowb = (unsigned)a.W * (unsigned)sizeof(float2);
+    st.row_ld = wrapi(tau0, a.H);
+    st.load_row(0, a.H, xoff);
+    st.load_row(1, a.H, xoff);
+    int tau = tau0;
+    for (; tau + U - 1 <= tau1; tau += U)
+        st.block(std::make_integer_sequence<int, U>{}, a, tau, r0, r1, xoff, ocol, out_lane, tau1);
+    if (tau <= tau1)
+        st.tail(std::make_integer_sequence<int, U - 1>{}, tau1 - tau + 1, a, tau, r0, r1, xoff, ocol, out_lane, tau1);
+
+    const double s_ls1 = wave_sum((double)st.acc_ls1);
+    const double s_ls2 = wave_sum((double)st.acc_ls2);
+    const double s_rs = wave_sum((double)st.acc_rs);
+    const double s_l1 = wave_sum((double)st.acc_l1);
+    const double s_tv = wave_sum((double)st.acc_tv);
+    const double s_nnz = wave_sum((double)st.acc_nnz);
+    if (lane == 0) {
+        double* p = a.partial + (size_t)w * PS_COUNT;
+        p[PS_LS1] = s_ls1;
+        p[PS_LS2] = s_ls2;
+        p[PS_RESTART] = s_rs;
+        p[PS_L1X0] = s_l1;
+        p[PS_TVX0] = s_tv;
+        p[PS_NNZX0] = s_nnz;
+        p[PS_NNZY] = (double)st.nnzy;
         p[7] = 0.0;
     }
 }
@@ -582,6 +814,83 @@ hipError_t prox_fl2d(const ProxLaunch& a, hipStream_t s) {
         case 10: return launch_fl2d<10>(d, s);
         default: return hipErrorInvalidValue;
     }
+}
+
+template <int NTV> static hipError_t launch_dense(const ProxDev& d, hipStream_t s) {
+    dim3 grid((d.nwaves + kProxWaves - 1) / kProxWaves);
+    hipLaunchKernelGGL(k_prox_fl2d_dense<NTV>, grid, dim3(64 * kProxWaves), 0, s, d);
+    return hipGetLastError();
+}
+
+hipError_t prox_fl2d_dense(const ProxLaunch& a, hipStream_t s) {
+    if ((size_t)a.W * a.H * sizeof(float2) > 0xffffffffull) return hipErrorInvalidValue;  // 32-bit row offsets
+    const ProxDev d = make_dev(a);
+    switch (a.n_tv) {
+        case 0: return launch_dense<0>(d, s);
+        case 1: return launch_dense<1>(d, s);
+        case 2: return launch_dense<2>(d, s);
+        case 3: return launch_dense<3>(d, s);
+        case 4: return launch_dense<4>(d, s);
+        case 5: return launch_dense<5>(d, s);
+        case 6: return launch_dense<6>(d, s);
+        case 7: return launch_dense<7>(d, s);
+        case 8: return launch_dense<8>(d, s);
+        case 9: return launch_dense<9>(d, s);
+        case 10: return launch_dense<10>(d, s);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+template <int NTV> static int dense_blocks_per_cu() {
+    int nb = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_prox_fl2d_dense<NTV>, 64 * kProxWaves, 0) != hipSuccess)
+        return 0;
+    return nb;
+}
+
+// The chunk length of least cost: rounds of resident waves, each of (rows + halo) steps whose time
+// is 0.18 + 0.45 w us with w waves on a SIMD and at least 0.65 (measured at n_tv = 5 over 64^2 x 8
+// ... 1024^2 x 16; only the ratios matter here).  Few waves take short chunks although each
+// re-reads 2 n_tv + 1 rows: 6 rows against 32 at 64^2 x 8 16 us against 32, 24 against 128 at
+// 256^2 x 32 36 against 93; at 512^2 x 100, where the device is full, 171 rows 263 us, 32 276.
+int prox_fl2d_dense_auto_rows(int W, int H, int nz, int n_tv) {
+    int nb = 0;
+    switch (n_tv) {
+        case 0: nb = dense_blocks_per_cu<0>(); break;
+        case 1: nb = dense_blocks_per_cu<1>(); break;
+        case 2: nb = dense_blocks_per_cu<2>(); break;
+        case 3: nb = dense_blocks_per_cu<3>(); break;
+        case 4: nb = dense_blocks_per_cu<4>(); break;
+        case 5: nb = dense_blocks_per_cu<5>(); break;
+        case 6: nb = dense_blocks_per_cu<6>(); break;
+        case 7: nb = dense_blocks_per_cu<7>(); break;
+        case 8: nb = dense_blocks_per_cu<8>(); break;
+        case 9: nb = dense_blocks_per_cu<9>(); break;
+        case 10: nb = dense_blocks_per_cu<10>(); break;
+        default: return 0;
+    }
+    int dev = 0, cus = 0;
+    if (nb <= 0 || hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+        return 0;
+    const double simds = 4.0 * cus;
+    const long slots = (long)nb * kProxWaves * cus;
+    const long strips = (long)prox_geom(W, H, n_tv, H).nstrips * nz;
+    auto step_us = [&](long waves) { return std::max(0.65, 0.18 + 0.45 * (double)waves / simds); };
+    double best_cost = 0;
+    int best_rc = 0;
+    for (int nch = 1; nch <= H; ++nch) {
+        const int rc = (H + nch - 1) / nch;
+        if (rc < kMinRowChunk && nch > 1) break;
+        const long waves = strips * ((H + rc - 1) / rc);
+        const double t = (double)(waves / slots) * step_us(slots) + (waves % slots ? step_us(waves % slots) : 0.0);
+        const double cost = t * (rc + 2 * n_tv + 1);
+        if (best_rc == 0 || cost < best_cost) {  // ties keep the longer chunk (less halo)
+            best_cost = cost;
+            best_rc = rc;
+        }
+    }
+    return best_rc;
 }
 
 // ----------------------------------------------------------------------------

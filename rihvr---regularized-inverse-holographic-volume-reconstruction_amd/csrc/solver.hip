@@ -27,6 +27,13 @@ namespace {
 
 constexpr double kPi = 3.14159265358979323846;
 
+// The non-zero fraction of y_{k-1} from which the mode-7 prox takes its dense form.  That form
+// costs the same for any content, but leaves its output without a line map, so A's column pass
+// then reads every line.  Prox + column pass per iteration with a line at 4 %, 10 % and never:
+// 599, 620, 679 us (1024^2 x 40, 66 % -> 5 % over 30 iterations), 557, 559, 587 (38 % -> 2 %),
+// 358, 385, 512 (512^2 x 100, 97 % -> 10 %); at 1 %, 598, 595 and 361.
+constexpr double kDenseFraction = 0.05;
+
 // scalar slots after reduction
 enum Slot { SL_PROX = 0, SL_RESID_A = 8, SL_RESID_M = 9, SL_COUNT = 16 };
 
@@ -81,6 +88,7 @@ struct SolveState {
     int total_bt = 0;
     int iters = 0;
     bool g_ready = false;     // G = A^T r of the current residual (else only R-hat is)
+    double nnz_y = 0;         // non-zero voxels of y_{k-1} (mode 7; 0 before the first prox)
 };
 
 }  // namespace
@@ -144,6 +152,7 @@ struct rihvr_ctx {
     int n_groups = 1;
     bool groups_one_stream = false;  // run A^T, prox and A group by group on the main stream
     int prox_rows = 0;    // output rows per prox wave (0: default)
+    int prox_rows_dense = 0;  // the same for the dense prox
     // Captured iterations: the two halves of a queued-ahead iteration (prox + A, then the
     // hologram momentum + the next A^T) as HIP graphs, one per pointer and step combination
     // (the volume ring, the maps and the spectra rotate through at most 12), replayed with the
@@ -157,6 +166,7 @@ struct rihvr_ctx {
         hipGraphExec_t exec;
     };
     std::vector<CachedGraph> gcache[2];
+    bool dense_ok = false;  // mode 7 with the fused prox on one stream: dense iterates take its dense form
     bool have_result = false;
     bool force_step = false;
     double forced_step = 0;
@@ -474,7 +484,8 @@ bool tv3d(const rihvr_ctx* c) { return c->ss.mode == RIHVR_MODE_FASTA_FUSED_LASS
 // enqueue = false performs only the host-side bookkeeping of the maps (a replayed graph holds
 // the launches)
 rihvr_status apply_prox(rihvr_ctx* c, int mode, const float2* Y0, const float2* YM, float s_mom, const float2* G,
-                        double t, float2* Y, const float* s_mom_dev = nullptr, bool enqueue = true) {
+                        double t, float2* Y, const float* s_mom_dev = nullptr, bool enqueue = true,
+                        bool dense = false) {
     ProxLaunch a;
     a.Y0 = Y0; a.YM = YM; a.G = G; a.Y = Y;
     a.W = c->W; a.H = c->H; a.nz = c->Nz;
@@ -491,6 +502,11 @@ rihvr_status apply_prox(rihvr_ctx* c, int mode, const float2* Y0, const float2* 
         // more TV iterations than the fused kernel holds: the multi-pass form (no maps)
         if (enqueue) RIHVR_TRY(timed(c, K_PROX, [&] { return prox_tv2_general(a, c->tvbuf, c->stream); }));
         rows = prox_tv2_num_blocks(c->W, c->H, c->Nz);
+        if (ky >= 0) c->occ_valid[ky] = false;
+    } else if (mode == RIHVR_MODE_FASTA_FUSED_LASSO_2D && dense) {
+        a.row_chunk = c->prox_rows_dense;
+        if (enqueue) RIHVR_TRY(timed(c, K_PROX, [&] { return prox_fl2d_dense(a, c->stream); }));
+        rows = prox_fl2d_num_waves(c->W, c->H, c->Nz, a.n_tv, c->prox_rows_dense);
         if (ky >= 0) c->occ_valid[ky] = false;
     } else if (mode == RIHVR_MODE_FASTA_FUSED_LASSO_2D) {
         // the new map is built in occ_tmp, then becomes Y's; a volume without a valid map
@@ -704,11 +720,17 @@ rihvr_status create_impl(const rihvr_params* params, const rihvr_schedule* sch, 
     RIHVR_TRY(dalloc(&c->twiW, c->W));
     RIHVR_TRY(dalloc(&c->twfH, c->H));
     RIHVR_TRY(dalloc(&c->twiH, c->H));
+    c->dense_ok = params->mode == RIHVR_MODE_FASTA_FUSED_LASSO_2D && !tv_general && c->n_groups == 1;
+    c->prox_rows_dense = c->prox_rows;
+    if (c->dense_ok && prow < 0)
+        c->prox_rows_dense = prox_fl2d_dense_auto_rows(c->W, c->H, c->Nz, params->num_tv_iterations);
     long rows = std::max<long>(prox_fl2d_num_waves(c->W, c->H, c->Nz, std::min(params->num_tv_iterations, 10), c->prox_rows),
                                prox_l1_num_blocks(c->W, c->H, c->Nz));
     rows = std::max<long>(rows, prox_fl3d_num_blocks(c->W, c->H, c->Nz));
     rows = std::max<long>(rows, momentum_out_num_blocks(c->W, c->H, c->Nz));
     rows = std::max<long>(rows, prox_tv2_num_blocks(c->W, c->H, c->Nz));
+    if (c->dense_ok)
+        rows = std::max<long>(rows, prox_fl2d_num_waves(c->W, c->H, c->Nz, params->num_tv_iterations, c->prox_rows_dense));
     c->partial_rows = rows;
     RIHVR_TRY(dalloc(&c->partial, (size_t)rows * PS_COUNT));
     c->holo_rows = std::max<long>(std::max<long>(holo_num_blocks(c->N), c->W / 16), holo_spec_num_blocks(c->W, c->H));
@@ -946,6 +968,7 @@ rihvr_status iterate_impl(rihvr_ctx* c, int n_it, rihvr_stats* st, bool last_f_b
         float2* Y0 = c->Yb[c->iy0];
         float2* YM = c->Yb[c->iym];
         bool queued = false;  // the accepted-iteration work is queued
+        const bool dense = c->dense_ok && s.nnz_y >= kDenseFraction * (double)c->V;
         for (;;) {
             const bool use_graph = ahead && c->graphs && !c->tm.on;
             if (!s.g_ready && mode == RIHVR_MODE_FASTA_FUSED_LASSO_2D && c->n_groups > 1) {
@@ -959,16 +982,16 @@ rihvr_status iterate_impl(rihvr_ctx* c, int n_it, rihvr_stats* st, bool last_f_b
                     const std::vector<const void*> key = {
                         Y0, YM, Yn, c->G, c->hX, c->occ[0], c->occ[1], c->occ[2], c->occ_tmp,
                         (const void*)(intptr_t)(c->occ_valid[0] | (c->occ_valid[1] << 1) | (c->occ_valid[2] << 2)),
-                        (const void*)(intptr_t)mode, (const void*)(uintptr_t)weight_bits(c)};
+                        (const void*)(intptr_t)(mode | (dense ? 256 : 0)), (const void*)(uintptr_t)weight_bits(c)};
                     RIHVR_TRY(graph_run(
                         c, 0, key, s.t,
                         [&] {
-                            RIHVR_TRY(apply_prox(c, mode, Y0, YM, s.s_mom, c->G, s.t, Yn, c->d_smom, true));
+                            RIHVR_TRY(apply_prox(c, mode, Y0, YM, s.s_mom, c->G, s.t, Yn, c->d_smom, true, dense));
                             return apply_forward(c, Yn, c->hX);
                         },
-                        [&] { return apply_prox(c, mode, Y0, YM, s.s_mom, c->G, s.t, Yn, c->d_smom, false); }));
+                        [&] { return apply_prox(c, mode, Y0, YM, s.s_mom, c->G, s.t, Yn, c->d_smom, false, dense); }));
                 } else {
-                    RIHVR_TRY(apply_prox(c, mode, Y0, YM, s.s_mom, c->G, s.t, Yn));
+                    RIHVR_TRY(apply_prox(c, mode, Y0, YM, s.s_mom, c->G, s.t, Yn, nullptr, true, dense));
                     RIHVR_TRY(apply_forward(c, Yn, c->hX));
                 }
             }
@@ -1069,6 +1092,7 @@ rihvr_status iterate_impl(rihvr_ctx* c, int n_it, rihvr_stats* st, bool last_f_b
             break;
         }
         if (i == n_it) break;  // stopped at the objective target
+        s.nnz_y = c->h_scal[SL_PROX + PS_NNZY];
         const double rs = c->h_scal[SL_PROX + PS_RESTART];
         const bool restart = rs > 0;  // :4481
         if (restart) alpha0 = 1;
