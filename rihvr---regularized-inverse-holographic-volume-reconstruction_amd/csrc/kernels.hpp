@@ -15,6 +15,8 @@ namespace rihvr {
 
 // ---- FFT (fft_kernels.hip) -------------------------------------------------
 bool fft_length_supported(int L);
+// workgroups of a row pass over one chunk of planes of H rows of length L (0: no fixed plan)
+int fft_rows_blocks(int L, int H);
 
 // Plain row FFT of nrows contiguous rows of length L.  tw: W_L^m for the sign.
 hipError_t fft_rows_plain(int L, int sign, const float2* in, float2* out, int nrows,
@@ -114,9 +116,9 @@ struct ProxLaunch {
 // row_chunk: output rows per wave (<= 0: default 128)
 int prox_fl2d_num_waves(int W, int H, int nz, int n_tv, int row_chunk);
 // Output rows per wave for this geometry on the current device: about 205 when that gives
-// at least two rounds of resident waves, else the chunk length whose rounds of resident
-// waves (rounded up) times the rows a wave steps through (its chunk plus the 2 n_tv + 1
-// halo rows) is least.  0 if the occupancy query fails.
+// at least two rounds of resident waves, else the chunk length of least estimated time (rounds of
+// resident waves, each of its chunk plus the 2 n_tv + 1 halo rows).  0 if the occupancy query
+// fails.
 int prox_fl2d_auto_rows(int W, int H, int nz, int n_tv);
 bool prox_fl2d_supported(int n_tv);
 hipError_t prox_fl2d(const ProxLaunch& a, hipStream_t s);

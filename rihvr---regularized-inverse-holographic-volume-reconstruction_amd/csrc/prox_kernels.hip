@@ -749,6 +749,26 @@ template <int NTV> static int fl2d_blocks_per_cu() {
     return nb;
 }
 
+// Output rows per wave of least cost for `strips` strips of H rows: rounds of `slots` resident
+// waves, each (rows + 2 n_tv + 1) steps of a + b w us, and at least `least`, with w waves on a SIMD.
+static int cheapest_rows(long strips, int H, int n_tv, long slots, int cus, double a, double b, double least) {
+    auto step = [&](long waves) { return std::max(least, a + b * (double)waves / (4.0 * cus)); };
+    double best_cost = 0;
+    int best_rc = 0;
+    for (int nch = 1; nch <= H; ++nch) {
+        const int rc = (H + nch - 1) / nch;
+        if (rc < kMinRowChunk && nch > 1) break;
+        const long waves = strips * ((H + rc - 1) / rc);
+        const double t = (double)(waves / slots) * step(slots) + (waves % slots ? step(waves % slots) : 0.0);
+        const double cost = t * (rc + 2 * n_tv + 1);
+        if (best_rc == 0 || cost < best_cost) {  // ties keep the longer chunk (less halo)
+            best_cost = cost;
+            best_rc = rc;
+        }
+    }
+    return best_rc;
+}
+
 int prox_fl2d_auto_rows(int W, int H, int nz, int n_tv) {
     int nb = 0;
     switch (n_tv) {
@@ -774,25 +794,13 @@ int prox_fl2d_auto_rows(int W, int H, int nz, int n_tv) {
     // Chunks of about 205 rows when they give at least two rounds of resident waves: waves
     // with data run longer, and the dispatcher balances them only over several rounds (on
     // MI355X at 1024^2 x 128, 205 rows was best or tied-best with 3, 4 and 5 waves per SIMD,
-    // and one round of 512-row chunks 7 % slower).  Smaller problems take the chunk that
-    // fills the device in the fewest rounds of the shortest waves.
+    // and one round of 512-row chunks 7 % slower).  Smaller problems take the chunk of least cost:
+    // rounds of resident waves, each of (rows + halo) steps whose time is 1.7 + 0.35 w us with w
+    // waves on a SIMD (measured on rows full of data: 64^2 x 8 25 us with 4 rows against 72 with 32,
+    // 256^2 x 32 67 with 8 against 97 with 32, 512^2 x 20 115 with 24 against 125 with 32).
     const int nch_target = std::max(1, (H + 102) / 205);
     if ((long)nstrips * nch_target * nz >= 2 * slots) return (H + nch_target - 1) / nch_target;
-    long best_cost = -1;
-    int best_rc = 0;
-    for (int nch = 1; nch <= H; ++nch) {
-        const int rc = (H + nch - 1) / nch;
-        if (rc < 32 && nch > 1) break;
-        const int chunks = (H + rc - 1) / rc;
-        const long waves = (long)nstrips * chunks * nz;
-        const long rounds = (waves + slots - 1) / slots;
-        const long cost = rounds * (rc + 2 * n_tv + 1);
-        if (best_cost < 0 || cost < best_cost) {  // ties keep the longer chunk (less halo)
-            best_cost = cost;
-            best_rc = rc;
-        }
-    }
-    return best_rc;
+    return cheapest_rows((long)nstrips * nz, H, n_tv, slots, cus, 1.7, 0.35, 0.0);
 }
 
 hipError_t prox_fl2d(const ProxLaunch& a, hipStream_t s) {
@@ -848,9 +856,8 @@ template <int NTV> static int dense_blocks_per_cu() {
     return nb;
 }
 
-// The chunk length of least cost: rounds of resident waves, each of (rows + halo) steps whose time
-// is 0.18 + 0.45 w us with w waves on a SIMD and at least 0.65 (measured at n_tv = 5 over 64^2 x 8
-// ... 1024^2 x 16; only the ratios matter here).  Few waves take short chunks although each
+// The chunk length of least cost, a step taking 0.18 + 0.45 w us with w waves on a SIMD and at least
+// 0.65 (measured at n_tv = 5 over 64^2 x 8 ... 1024^2 x 16; only the ratios matter here).  Few waves take short chunks although each
 // re-reads 2 n_tv + 1 rows: 6 rows against 32 at 64^2 x 8 16 us against 32, 24 against 128 at
 // 256^2 x 32 36 against 93; at 512^2 x 100, where the device is full, 171 rows 263 us, 32 276.
 int prox_fl2d_dense_auto_rows(int W, int H, int nz, int n_tv) {
@@ -873,24 +880,8 @@ int prox_fl2d_dense_auto_rows(int W, int H, int nz, int n_tv) {
     if (nb <= 0 || hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         return 0;
-    const double simds = 4.0 * cus;
-    const long slots = (long)nb * kProxWaves * cus;
-    const long strips = (long)prox_geom(W, H, n_tv, H).nstrips * nz;
-    auto step_us = [&](long waves) { return std::max(0.65, 0.18 + 0.45 * (double)waves / simds); };
-    double best_cost = 0;
-    int best_rc = 0;
-    for (int nch = 1; nch <= H; ++nch) {
-        const int rc = (H + nch - 1) / nch;
-        if (rc < kMinRowChunk && nch > 1) break;
-        const long waves = strips * ((H + rc - 1) / rc);
-        const double t = (double)(waves / slots) * step_us(slots) + (waves % slots ? step_us(waves % slots) : 0.0);
-        const double cost = t * (rc + 2 * n_tv + 1);
-        if (best_rc == 0 || cost < best_cost) {  // ties keep the longer chunk (less halo)
-            best_cost = cost;
-            best_rc = rc;
-        }
-    }
-    return best_rc;
+    return cheapest_rows((long)prox_geom(W, H, n_tv, H).nstrips * nz, H, n_tv, (long)nb * kProxWaves * cus, cus, 0.18,
+                         0.45, 0.65);
 }
 
 // ----------------------------------------------------------------------------

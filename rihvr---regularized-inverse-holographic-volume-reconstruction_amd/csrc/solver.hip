@@ -166,7 +166,7 @@ struct rihvr_ctx {
         hipGraphExec_t exec;
     };
     std::vector<CachedGraph> gcache[2];
-    bool dense_ok = false;  // mode 7 with the fused prox on one stream: dense iterates take its dense form
+    bool dense_ok = false;  // mode 7 with the fused prox: dense iterates take its dense form
     bool have_result = false;
     bool force_step = false;
     double forced_step = 0;
@@ -546,7 +546,8 @@ rihvr_status apply_prox(rihvr_ctx* c, int mode, const float2* Y0, const float2* 
 // the main stream; the main stream waits for group g's G planes before its prox.
 // Same kernels, same arithmetic and the same partial-row layout as the one-stream
 // sequence A^T (all planes), prox (all planes), A (all planes).
-rihvr_status pipelined_pass(rihvr_ctx* c, const float2* Y0, const float2* YM, float s_mom, double t, float2* Yn) {
+rihvr_status pipelined_pass(rihvr_ctx* c, const float2* Y0, const float2* YM, float s_mom, double t, float2* Yn,
+                            bool dense) {
     if (!c->groups_one_stream) {
         RIHVR_HIP(hipStreamWaitEvent(c->aux, c->ev_rhat, 0));
         for (int g = 0, g0 = 0; g < c->n_groups; ++g, g0 += c->pipe_planes) {
@@ -560,13 +561,13 @@ rihvr_status pipelined_pass(rihvr_ctx* c, const float2* Y0, const float2* YM, fl
     a.reg = (double)c->p.regularization_param;
     a.reg_tv = (double)c->p.regularization_TV_param;
     a.n_tv = c->p.num_tv_iterations;
-    a.row_chunk = c->prox_rows;
-    const int per_plane = prox_fl2d_num_waves(c->W, c->H, 1, a.n_tv, c->prox_rows);
+    a.row_chunk = dense ? c->prox_rows_dense : c->prox_rows;
+    const int per_plane = prox_fl2d_num_waves(c->W, c->H, 1, a.n_tv, a.row_chunk);
     const uint64_t* o0 = occ_of(c, Y0);
     const uint64_t* om = occ_of(c, YM);
     const int ky = ring_index(c, Yn);
     const uint64_t* oold = (ky >= 0 && c->occ_valid[ky]) ? c->occ[ky] : c->occ_ones;
-    RIHVR_HIP(hipMemsetAsync(c->occ_tmp, 0, map_words(c) * sizeof(uint64_t), c->stream));
+    if (!dense) RIHVR_HIP(hipMemsetAsync(c->occ_tmp, 0, map_words(c) * sizeof(uint64_t), c->stream));
     for (int g = 0, g0 = 0; g < c->n_groups; ++g, g0 += c->pipe_planes) {
         const int gz = std::min(c->pipe_planes, c->Nz - g0);
         const size_t off = (size_t)g0 * c->N;
@@ -583,10 +584,12 @@ rihvr_status pipelined_pass(rihvr_ctx* c, const float2* Y0, const float2* YM, fl
         a.occ_old = oold + roff;
         a.occ_new = c->occ_tmp + roff;
         a.occ_new_planes = c->occ_tmp + (size_t)c->Nz * c->H + g0;
-        RIHVR_TRY(timed(c, K_PROX, [&] { return prox_fl2d(a, c->stream); }));
-        RIHVR_TRY(forward_group(c, Yn, g0, gz, c->stream, ky >= 0 ? c->occ_tmp : nullptr));
+        RIHVR_TRY(timed(c, K_PROX, [&] { return dense ? prox_fl2d_dense(a, c->stream) : prox_fl2d(a, c->stream); }));
+        RIHVR_TRY(forward_group(c, Yn, g0, gz, c->stream, ky >= 0 && !dense ? c->occ_tmp : nullptr));
     }
-    if (ky >= 0) {
+    if (ky >= 0 && dense) {
+        c->occ_valid[ky] = false;
+    } else if (ky >= 0) {
         std::swap(c->occ[ky], c->occ_tmp);
         c->occ_valid[ky] = true;
     }
@@ -639,6 +642,20 @@ rihvr_status check_schedule(const rihvr_schedule* s) {
     return ok ? RIHVR_OK : RIHVR_E_INVALID_ARGUMENT;
 }
 
+// Planes per workgroup of a row pass that has `blocks` workgroups per plane chunk: as many as
+// leave `target` workgroups, at most `most`, and at least 2 (1 where even single planes do not
+// fill the device).  A workgroup's planes are a serial chain (2.5 us each at L = 256), while more
+// chunks cost A more partial spectra to write and sum.  Forward row pass + spectrum sum, us, by
+// planes per chunk: 256^2 x 32 (16 workgroups a chunk) 2: 22, 8: 31, 32: 86; 512^2 x 100 (128)
+// 4: 75, 16: 62, 32: 87; 448^2 x 40 (112) 8: 40, 32: 83; 1024^2 x 16 (512) 4: 59, 16: 54.  A^T's:
+// 256^2 x 32 1: 11, 2: 12, 8: 25; 512^2 x 20 2: 18, 8: 21; 1024^2 x 16 4: 41, 8: 37.
+int split_planes(int nz, int blocks, int target, int most) {
+    const int chunks = (target + blocks - 1) / blocks;
+    const int zc = (nz + chunks - 1) / chunks;
+    const int least = (long)nz * blocks <= 256 ? 1 : 2;
+    return std::max(std::min(zc, most), least);
+}
+
 // sch: the launch choices (NULL: the defaults, with the RIHVR_* environment overrides)
 rihvr_status create_impl(const rihvr_params* params, const rihvr_schedule* sch, rihvr_ctx** out) {
     RIHVR_TRY(validate(params));
@@ -656,8 +673,9 @@ rihvr_status create_impl(const rihvr_params* params, const rihvr_schedule* sch, 
     RIHVR_HIP(hipStreamCreateWithFlags(&c->aux, hipStreamNonBlocking));
     RIHVR_HIP(hipEventCreateWithFlags(&c->ev_rhat, hipEventDisableTiming));
     RIHVR_HIP(hipEventCreateWithFlags(&c->ev_scal, hipEventDisableTiming));
-    // defaults: A's partial spectra over 32 planes; A^T's row pass walks 8 planes per workgroup
-    // (at 1024^2 x 128: 588 against 584 iter/s with 16 over whole solves, the same bits)
+    // With a schedule: A's partial spectra over 32 planes, A^T's row pass over 8 planes per
+    // workgroup, where its fields are 0.  Without one, split_planes gives small problems more and
+    // shorter chunks.
     int zc = 32, za = 8, prow = -1;
     bool force_gen = false;
     if (sch) {
@@ -668,6 +686,10 @@ rihvr_status create_impl(const rihvr_params* params, const rihvr_schedule* sch, 
         force_gen = sch->fft_path == 1;
         c->graphs = sch->graphs != 0;
     } else {
+        if (fft_length_supported(c->W) && fft_length_supported(c->H)) {
+            zc = split_planes(c->Nz, fft_rows_blocks(c->W, c->H), 640, 32);
+            za = split_planes(c->Nz, fft_rows_blocks(c->W, c->H), 1024, 8);
+        }
         if (const char* e = std::getenv("RIHVR_ZCHUNK")) zc = std::max(1, std::atoi(e));
         if (const char* e = std::getenv("RIHVR_ZCHUNK_ADJ")) za = std::max(1, std::atoi(e));
         if (const char* e = std::getenv("RIHVR_PROX_ROWS")) prow = std::max(0, std::atoi(e));
@@ -720,9 +742,11 @@ rihvr_status create_impl(const rihvr_params* params, const rihvr_schedule* sch, 
     RIHVR_TRY(dalloc(&c->twiW, c->W));
     RIHVR_TRY(dalloc(&c->twfH, c->H));
     RIHVR_TRY(dalloc(&c->twiH, c->H));
-    c->dense_ok = params->mode == RIHVR_MODE_FASTA_FUSED_LASSO_2D && !tv_general && c->n_groups == 1;
+    c->dense_ok = params->mode == RIHVR_MODE_FASTA_FUSED_LASSO_2D && !tv_general;
     c->prox_rows_dense = c->prox_rows;
-    if (c->dense_ok && prow < 0)
+    // rows that a schedule gives hold for both forms, except where they are the rule's own (a
+    // schedule read back from a context)
+    if (c->dense_ok && (prow < 0 || prow == prox_fl2d_auto_rows(c->W, c->H, c->Nz, params->num_tv_iterations)))
         c->prox_rows_dense = prox_fl2d_dense_auto_rows(c->W, c->H, c->Nz, params->num_tv_iterations);
     long rows = std::max<long>(prox_fl2d_num_waves(c->W, c->H, c->Nz, std::min(params->num_tv_iterations, 10), c->prox_rows),
                                prox_l1_num_blocks(c->W, c->H, c->Nz));
@@ -972,7 +996,7 @@ rihvr_status iterate_impl(rihvr_ctx* c, int n_it, rihvr_stats* st, bool last_f_b
         for (;;) {
             const bool use_graph = ahead && c->graphs && !c->tm.on;
             if (!s.g_ready && mode == RIHVR_MODE_FASTA_FUSED_LASSO_2D && c->n_groups > 1) {
-                RIHVR_TRY(pipelined_pass(c, Y0, YM, s.s_mom, s.t, Yn));
+                RIHVR_TRY(pipelined_pass(c, Y0, YM, s.s_mom, s.t, Yn, dense));
             } else {
                 if (!s.g_ready)
                     for (int g0 = 0; g0 < c->Nz; g0 += c->pipe_planes)
