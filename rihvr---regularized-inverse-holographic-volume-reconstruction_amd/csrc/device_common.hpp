@@ -71,6 +71,16 @@ __device__ __forceinline__ float2 transfer(double z, double kappa) {
     return make_float2(c, s);
 }
 
+// --- placement on the 8 XCDs -----------------------------------------------
+// Bijection of [0, nblocks): block b, which the hardware places on XCD b % 8, gets the
+// logical index of the (b / 8)-th block of a contiguous run assigned to that XCD.
+constexpr int kXcds = 8;
+__device__ __forceinline__ int xcd_local_block(int b, int nblocks) {
+    const int q = nblocks / kXcds, r = nblocks % kXcds;
+    const int x = b % kXcds, k = b / kXcds;
+    return (x < r) ? x * (q + 1) + k : r * (q + 1) + (x - r) * q + k;
+}
+
 // --- wave64 / workgroup reductions in double ---------------------------------
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll

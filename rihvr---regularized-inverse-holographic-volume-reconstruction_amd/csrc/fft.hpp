@@ -19,9 +19,8 @@ namespace rihvr {
 
 // ---------------------------------------------------------------------------
 // Radix plans.  TPT = L / R0 threads per transform (one first-pass butterfly
-// per thread).  Radices 2, 4, 8, 16 have hand-written butterflies; any other
-// radix (3, 5, 7, 9, 13) uses a direct DFT with roots read from the twiddle
-// table (W_R^m = W_L^{m L / R}).
+// per thread).  Radices 2, 4, 8, 16, 32 have hand-written butterflies; the odd ones
+// (3, 5, 7, 9, 11, 13) a direct DFT with constant roots.
 // ---------------------------------------------------------------------------
 template <int... R> struct Radices {};
 
@@ -201,22 +200,56 @@ template <int SIGN, int L> struct Dft<32, SIGN, L> {
         combine(v, e, o, std::make_integer_sequence<int, 16>{});
     }
 };
-// generic direct DFT (odd radices); roots from the L-point twiddle table
-template <int R, int SIGN, int L> struct Dft {
-    __device__ static __forceinline__ void run(float2 (&v)[R], const float2* tw) {
-        float2 o[R];
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
-            float2 acc = v[0];
-#pragma unroll
-            for (int r = 1; r < R; ++r) {
-                float2 w = tw[((r * k) % R) * (L / R)];
-                acc = cadd(acc, cmul(v[r], w));
-            }
-            o[k] = acc;
+// cos and sin of 2 pi m / R as constants: the power series on [-pi, pi], in double
+constexpr double ct_pi = 3.14159265358979323846;
+constexpr double ct_series(double x, bool sine) {
+    double term = sine ? x : 1.0, sum = term;
+    for (int n = sine ? 2 : 1; n < 40; n += 2) {
+        term *= -x * x / ((double)n * (n + 1));
+        sum += term;
+    }
+    return sum;
+}
+template <int R> struct Roots {
+    float c[R], s[R];
+    constexpr Roots() : c(), s() {
+        for (int m = 0; m < R; ++m) {
+            const double x = 2.0 * ct_pi * (2 * m > R ? m - R : m) / R;
+            c[m] = (float)ct_series(x, false);
+            s[m] = (float)ct_series(x, true);
         }
+    }
+};
+// Odd radices: the inputs j and R - j in pairs, x_j w + x_{R-j} conj(w) = (x_j + x_{R-j}) cos
+// + i (x_j - x_{R-j}) sin, and outputs k and R - k from the same two sums: (R - 1)^2 real products
+// of constants instead of (R - 1)^2 complex ones with roots read from the twiddle table.
+template <int R, int SIGN, int L> struct Dft {
+    static_assert(R % 2 == 1, "the even radices have their own butterflies");
+    __device__ static __forceinline__ void run(float2 (&v)[R], const float2*) {
+        constexpr Roots<R> w{};
+        constexpr int h = (R - 1) / 2;
+        float2 a[h], b[h];
+        float2 sum = v[0];
 #pragma unroll
-        for (int k = 0; k < R; ++k) v[k] = o[k];
+        for (int j = 0; j < h; ++j) {
+            a[j] = cadd(v[j + 1], v[R - 1 - j]);
+            b[j] = csub(v[j + 1], v[R - 1 - j]);
+            sum = cadd(sum, a[j]);
+        }
+        const float2 x0 = v[0];
+        v[0] = sum;
+#pragma unroll
+        for (int k = 1; k <= h; ++k) {
+            float2 p = x0, q = make_float2(0.0f, 0.0f);
+#pragma unroll
+            for (int j = 0; j < h; ++j) {
+                const float c = w.c[((j + 1) * k) % R], s = SIGN < 0 ? -w.s[((j + 1) * k) % R] : w.s[((j + 1) * k) % R];
+                p = make_float2(fmaf(a[j].x, c, p.x), fmaf(a[j].y, c, p.y));
+                q = make_float2(fmaf(b[j].x, s, q.x), fmaf(b[j].y, s, q.y));
+            }
+            v[k] = make_float2(p.x - q.y, p.y + q.x);
+            v[R - k] = make_float2(p.x + q.y, p.y - q.x);
+        }
     }
 };
 

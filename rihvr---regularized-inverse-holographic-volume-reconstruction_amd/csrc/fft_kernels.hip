@@ -275,6 +275,7 @@ struct ColArgs {
     const uint64_t* occ;
     const uint64_t* occ_planes;
     uint8_t* smap;
+    int lsh;                // a line is 2^lsh columns
 };
 
 template <int L, int SIGN, int MODE>
@@ -284,7 +285,7 @@ __global__ void __launch_bounds__((ColCfg<L, MODE>::THREADS)) k_cols(ColArgs a) 
     if constexpr (MODE == COL_FWD) {
         // a strip with no line set in its plane transforms to zeros: not written, and the
         // workgroup leaves before anything else (uniform: every thread reads the same word)
-        if (a.occ_planes && !((a.occ_planes[blockIdx.y] >> blockIdx.x) & 1ull)) {
+        if (a.occ_planes && !((a.occ_planes[blockIdx.y] >> ((blockIdx.x * kColStrip) >> a.lsh)) & 1ull)) {
             if (threadIdx.x == 0) a.smap[(size_t)blockIdx.y * (a.W / kColStrip) + blockIdx.x] = 0;
             return;
         }
@@ -316,11 +317,11 @@ __global__ void __launch_bounds__((ColCfg<L, MODE>::THREADS)) k_cols(ColArgs a) 
             lds);
     } else if constexpr (MODE == COL_FWD) {
         // A, first pass: x_z e^{-i phi_z} (sparse_phase_scale_kernel with -z), forward column FFT.
-        // The workgroup's 16 columns are line blockIdx.x of every row: rows whose line is
+        // The workgroup's 16 columns lie in one line of every row: rows whose line is
         // empty are not read, and a strip empty in every row transforms to zeros, which are
         // not written (the strip map tells the row pass).
         const int z = blockIdx.y;
-        const int line = blockIdx.x;
+        const int line = (blockIdx.x * kColStrip) >> a.lsh;
         const uint64_t* occ = a.occ ? a.occ + (size_t)z * L : nullptr;
         // the strip's row bits in LDS (from the map, or all set without one)
         __shared__ uint32_t rows_s[(L + 31) / 32];
@@ -335,7 +336,7 @@ __global__ void __launch_bounds__((ColCfg<L, MODE>::THREADS)) k_cols(ColArgs a) 
                 }
         }
         const bool any = occ ? __syncthreads_or(mine) : true;
-        if (threadIdx.x == 0) a.smap[(size_t)z * (W / kColStrip) + line] = any ? 1 : 0;
+        if (threadIdx.x == 0) a.smap[(size_t)z * (W / kColStrip) + blockIdx.x] = any ? 1 : 0;
         if (!any) return;  // uniform: the whole workgroup leaves
         const float2 ph = a.phase[z];
         const float px = ph.x, py = -ph.y;
@@ -492,7 +493,7 @@ hipError_t fft_cols_fwd(int L, const float2* in, const float2* phase, float2* ou
                         hipStream_t s) {
     ColArgs a{};
     a.in = in; a.out = out; a.W = W; a.twg = tw_fwd; a.phase = phase; a.occ = occ; a.occ_planes = occ_planes;
-    a.smap = smap;
+    a.smap = smap; a.lsh = line_shift(W);
     switch (L) {
 #define X(n) case n: return launch_cols_t<n, -1, COL_FWD>(a, nz, s);
         RIHVR_FOR_EACH_L(X)

@@ -8,10 +8,15 @@ namespace rihvr {
 // Line occupancy of a prox-output volume: one 64-bit word per (plane, row), bit l set when
 // the row's voxels l L .. l L + L - 1 hold a non-zero value, L = 16 voxels (one 128-byte line)
 // for W <= 1024, else the least power of two giving at most 64 lines (32 up to 2048, 64 up to
-// 4096; only the fixed-length FFT kernels, W <= 1024, read the maps besides the prox).  A
-// volume with a valid map holds exact zeros in every line whose bit is clear, so readers
+// 4096).  A volume with a valid map holds exact zeros in every line whose bit is clear, so readers
 // may skip those lines and writers may skip zero lines that were already zero.  A map is
 // [nz][H] row words followed by [nz] plane words, each the OR of its plane's row words.
+
+inline int line_shift(int W) {  // log2 L
+    int lsh = 4;
+    while (((W - 1) >> lsh) >= 64) ++lsh;
+    return lsh;
+}
 
 // ---- FFT (fft_kernels.hip) -------------------------------------------------
 bool fft_length_supported(int L);
@@ -52,27 +57,29 @@ hipError_t fft_cols_adj(int L, const float2* in, const float2* phase, float2* ou
 hipError_t fft_cols_real(int L, const float2* in, float2* est, const float2* meas, float2* resid,
                          double* partial, int W, const float2* tw_inv, hipStream_t s);
 
-// ---- FFTs of any length 2..4096 (fft_generic.hip) -----------------------------------
-// Row transforms of length L with a plan chosen at run time; transforms along y run between
-// tiled transposes ([z][R][C] -> [z][C][R]).  Same roles as the fixed-length launchers above.
+// ---- FFTs of run-time length, multiples of 16 up to 4096 (fft_generic.hip) ------------
+// The launchers above with a plan chosen at run time; radix: the plan's largest (16, 8 or 4; an
+// autotuner choice).
 bool gen_fft_supported(int L);
-// max_radix: the largest radix of the plan (16, 8 or 4; an autotuner choice)
-hipError_t gen_rows_plain(int L, int sign, const float2* in, float2* out, long nrows, const float2* tw, hipStream_t s,
-                          int max_radix = 16);
-hipError_t gen_rows_sumparts(int L, const float2* parts, int nparts, long part_stride, float2* out, int nrows,
-                             const float2* tw_inv, hipStream_t s, int max_radix = 16);
-hipError_t gen_rows_adj(int L, const float2* rhat, const double* kappa, const float* zlist, float2* out, int nrows,
-                        int nz, int zchunk, float invN, const float2* tw_inv, hipStream_t s, int max_radix = 16);
-hipError_t gen_rows_fwdacc(int L, const float2* in, const double* kappa, const float* zlist, float2* parts, int nrows,
-                           int nz, int zchunk, const float2* tw_fwd, hipStream_t s, int max_radix = 16);
-// out[z][c][r] = in[z][r][c] (times phase[z], conjugated with conj; phase may be NULL)
-hipError_t gen_transpose(const float2* in, float2* out, int R, int C, int nz, const float2* phase, bool conj,
-                         hipStream_t s);
-// in [C][R] (a transposed estimate): est = (Re, 0) [R][C], resid = est - meas,
-// partial[block] = sum |resid|^2 over gen_transpose_real_blocks(R, C) blocks
-int gen_transpose_real_blocks(int R, int C);
-hipError_t gen_transpose_real(const float2* in, float2* est, const float2* meas, float2* resid, double* partial, int R,
-                              int C, hipStream_t s);
+int gen_rows_blocks(int L, int H);
+int gen_cols_blocks(int L, int W);  // workgroups of a column pass over one plane (partials of gen_cols_real)
+hipError_t gen_rows_plain(int L, int radix, int sign, const float2* in, float2* out, int nrows, const float2* tw,
+                          hipStream_t s);
+hipError_t gen_rows_sumparts(int L, int radix, const float2* parts, int nparts, long part_stride, float2* out,
+                             int nrows, const float2* tw_inv, hipStream_t s);
+hipError_t gen_rows_adj(int L, int radix, const float2* rhat, const double* kappa, const float* zlist, float2* out,
+                        int nrows, int nz, int zchunk, float invN, const float2* tw_inv, hipStream_t s);
+hipError_t gen_rows_fwdacc(int L, int radix, const float2* in, const double* kappa, const float* zlist, float2* parts,
+                           int nrows, int nz, int zchunk, const float2* tw_fwd, const uint8_t* smap, hipStream_t s);
+hipError_t gen_cols_plain(int L, int radix, int sign, const float2* in, float2* out, int W, int nplanes,
+                          const float2* tw, hipStream_t s);
+hipError_t gen_cols_adj(int L, int radix, const float2* in, const float2* phase, float2* out, int W, int nz,
+                        const float2* tw_inv, hipStream_t s);
+hipError_t gen_cols_fwd(int L, int radix, const float2* in, const float2* phase, float2* out, int W, int nz,
+                        const float2* tw_fwd, const uint64_t* occ, const uint64_t* occ_planes, uint8_t* smap,
+                        hipStream_t s);
+hipError_t gen_cols_real(int L, int radix, const float2* in, float2* est, const float2* meas, float2* resid,
+                         double* partial, int W, const float2* tw_inv, hipStream_t s);
 
 // ---- prox and elementwise (prox_kernels.hip) --------------------------------
 // Reduction slots written by the prox kernels (per wave partials, summed by reduce_partials).

@@ -55,15 +55,6 @@ int prox_fl2d_num_waves(int W, int H, int nz, int n_tv, int row_chunk) {
 }
 bool prox_fl2d_supported(int n_tv) { return n_tv >= 0 && n_tv <= kMaxNtv; }
 
-// Bijection of [0, nblocks): block b, which the hardware places on XCD b % 8, gets the
-// logical index of the (b / 8)-th block of a contiguous run assigned to that XCD.
-constexpr int kXcds = 8;
-__device__ __forceinline__ int xcd_local_block(int b, int nblocks) {
-    const int q = nblocks / kXcds, r = nblocks % kXcds;
-    const int x = b % kXcds, k = b / kXcds;
-    return (x < r) ? x * (q + 1) + k : r * (q + 1) + (x - r) * q + k;
-}
-
 struct ProxDev {
     const float2* Y0;
     const float2* YM;
@@ -723,8 +714,7 @@ static ProxDev make_dev(const ProxLaunch& a) {
     d.sc = a.reg_tv != 0.0 ? (float)(1 / (4 * 3 * a.t * a.reg_tv)) : 0.0f;
     d.thr = (float)(a.t * a.reg);
     d.do_soft = a.reg > 0.0;
-    d.lsh = 4;
-    while (((a.W - 1) >> d.lsh) >= 64) ++d.lsh;
+    d.lsh = line_shift(a.W);
     d.geo = prox_geom(a.W, a.H, a.n_tv, a.row_chunk);
     d.nwaves = d.geo.nstrips * d.geo.nchunks * a.nz;
     d.partial = a.partial;
@@ -1342,8 +1332,7 @@ hipError_t momentum_out(const float2* Y, const float2* Y0, float s_mom, float2* 
 
 hipError_t volume_terms_map(const float2* X, const uint64_t* occ, int W, int H, int nz, bool tv3d,
                             double* partial, hipStream_t s) {
-    int lsh = 4;
-    while (((W - 1) >> lsh) >= 64) ++lsh;
+    const int lsh = line_shift(W);
     dim3 grid(momentum_out_num_blocks(W, H, nz));
     hipLaunchKernelGGL(k_volume_terms<true>, grid, dim3(64 * kVtWaves), 0, s, X, X, 0.0f, (float2*)nullptr, W, H,
                        nz, tv3d ? 1 : 0, vt_rows_per_wave(W), occ, lsh, partial);
@@ -1533,8 +1522,7 @@ k_soft_map2(const float2* __restrict__ in, int W, int H, int nz, int rpw, int ls
 }
 hipError_t soft_threshold_map2(const float2* in, int W, int H, int nz, float tau0, float2* out0, uint64_t* occ0,
                                float tau1, float2* out1, uint64_t* occ1, hipStream_t s) {
-    int lsh = 4;
-    while (((W - 1) >> lsh) >= 64) ++lsh;
+    const int lsh = line_shift(W);
     hipLaunchKernelGGL(k_soft_map2, dim3(momentum_out_num_blocks(W, H, nz)), dim3(64 * kVtWaves), 0, s, in, W, H, nz,
                        vt_rows_per_wave(W), lsh, tau0, out0, occ0, tau1, out1, occ1);
     return hipGetLastError();

@@ -116,11 +116,10 @@ struct rihvr_ctx {
     float2* G = nullptr;                          // A^T r
     float2* G_alt = nullptr;                      // the next iteration's A^T r, formed ahead
     float2* T = nullptr;                          // FFT scratch volume
-    // FFTs of lengths outside the fixed-length kernels' set: rows with run-time plans between
-    // transposes (fft_generic.hip); T2 holds the transposed planes
-    bool gen = false;
-    int gen_radix = 16;  // the run-time plans' largest radix
-    float2* T2 = nullptr;
+    // FFTs of lengths outside the fixed-length kernels' set (or all, by the schedule) run with
+    // run-time plans (fft_generic.hip): the plans' largest radix along x and y, 0 for a fixed plan
+    int rad_w = 0, rad_h = 0;
+    int gen_radix = 16;  // the schedule's choice
     float2* tvbuf = nullptr;                      // 4 volumes for mode 7 with n_tv above the fused prox's limit
     float2* out = nullptr;                        // points at the returned volume
     // holograms
@@ -192,10 +191,8 @@ rihvr_status validate(const rihvr_params* p) {
     if (p->mode != RIHVR_MODE_FASTA_L1 && p->mode != RIHVR_MODE_FASTA_FUSED_LASSO &&
         p->mode != RIHVR_MODE_FASTA_FUSED_LASSO_2D)
         return RIHVR_E_INVALID_ARGUMENT;
-    // any length the fixed-length FFT kernels or the run-time plans cover (up to 4096)
-    if (!(fft_length_supported(p->width) && fft_length_supported(p->height)) &&
-        !(gen_fft_supported(p->width) && gen_fft_supported(p->height)))
-        return RIHVR_E_INVALID_ARGUMENT;
+    // the lengths that the run-time plans cover (the fixed ones among them)
+    if (!gen_fft_supported(p->width) || !gen_fft_supported(p->height)) return RIHVR_E_INVALID_ARGUMENT;
     return RIHVR_OK;
 }
 
@@ -334,28 +331,19 @@ void invalidate_occ(rihvr_ctx* c, const float2* v) {
 rihvr_status forward_group(rihvr_ctx* c, const float2* vol, int g0, int gz, hipStream_t st, const uint64_t* occ) {
     float2* Tg = c->T + (size_t)g0 * c->N;
     float2* spg = c->spart + (size_t)(g0 / c->zchunk_fwd) * c->N;
-    if (c->gen) {
-        // columns as rows of the transposed planes ([z][W][H]); every line is read
-        float2* Tt = c->T2 + (size_t)g0 * c->N;
-        RIHVR_TRY(timed_on(c, K_COLS_FWD, st, [&] {
-            hipError_t e = gen_transpose(vol + (size_t)g0 * c->N, Tt, c->H, c->W, gz, c->phase_fwd + g0, true, st);
-            if (e == hipSuccess) e = gen_rows_plain(c->H, -1, Tt, Tt, (long)gz * c->W, c->twfH, st, c->gen_radix);
-            if (e == hipSuccess) e = gen_transpose(Tt, Tg, c->W, c->H, gz, nullptr, false, st);
-            return e;
-        }));
-        return timed_on(c, K_ROWS_FWDACC, st, [&] {
-            return gen_rows_fwdacc(c->W, Tg, c->kappa, c->zlist + g0, spg, c->H, gz, c->zchunk_fwd, c->twfW, st, c->gen_radix);
-        });
-    }
     uint8_t* smg = c->smap + (size_t)g0 * (c->W / 16);
     const uint64_t* og = occ ? occ + (size_t)g0 * c->H : nullptr;
     const uint64_t* opg = occ ? map_planes(c, occ) + g0 : nullptr;
     RIHVR_TRY(timed_on(c, K_COLS_FWD, st, [&] {
-        return fft_cols_fwd(c->H, vol + (size_t)g0 * c->N, c->phase_fwd + g0, Tg, c->W, gz, c->twfH, og, opg, smg, st);
+        const float2 *v = vol + (size_t)g0 * c->N, *ph = c->phase_fwd + g0;
+        return c->rad_h ? gen_cols_fwd(c->H, c->rad_h, v, ph, Tg, c->W, gz, c->twfH, og, opg, smg, st)
+                        : fft_cols_fwd(c->H, v, ph, Tg, c->W, gz, c->twfH, og, opg, smg, st);
     }));
     RIHVR_TRY(timed_on(c, K_ROWS_FWDACC, st, [&] {
-        return fft_rows_fwdacc(c->W, Tg, c->kappa, c->zlist + g0, spg, c->H, gz, c->zchunk_fwd, c->twfW, smg,
-                               st);
+        return c->rad_w ? gen_rows_fwdacc(c->W, c->rad_w, Tg, c->kappa, c->zlist + g0, spg, c->H, gz, c->zchunk_fwd,
+                                          c->twfW, smg, st)
+                        : fft_rows_fwdacc(c->W, Tg, c->kappa, c->zlist + g0, spg, c->H, gz, c->zchunk_fwd, c->twfW,
+                                          smg, st);
     }));
     return RIHVR_OK;
 }
@@ -378,21 +366,16 @@ rihvr_status forward_finish(rihvr_ctx* c, float2* est) {
 // The spatial estimate and residual of a spectrum est_spec (FFT(est) / N): est = Re(IFFT(.)),
 // into hspat, and resid = est - meas (back_propagate_finish_kernel, RM_EST_TRUE)
 rihvr_status spatial_estimate(rihvr_ctx* c, const float2* est_spec) {
-    if (c->gen) {
-        RIHVR_TRY(timed(c, K_ROWS_SUMPARTS, [&] {
-            return gen_rows_sumparts(c->W, est_spec, 1, c->N, c->htmp, c->H, c->twiW, c->stream, c->gen_radix);
-        }));
-        return timed(c, K_COLS_REAL, [&] {
-            hipError_t e = gen_transpose(c->htmp, c->T2, c->H, c->W, 1, nullptr, false, c->stream);
-            if (e == hipSuccess) e = gen_rows_plain(c->H, 1, c->T2, c->T2, c->W, c->twiH, c->stream, c->gen_radix);
-            if (e == hipSuccess)
-                e = gen_transpose_real(c->T2, c->hspat, c->meas, c->resid, c->partial_holo, c->H, c->W, c->stream);
-            return e;
-        });
-    }
-    RIHVR_TRY(timed(c, K_ROWS_SUMPARTS, [&] { return fft_rows_sumparts(c->W, est_spec, 1, c->N, c->htmp, c->H, c->twiW, c->stream); }));
-    RIHVR_TRY(timed(c, K_COLS_REAL, [&] { return fft_cols_real(c->H, c->htmp, c->hspat, c->meas, c->resid, c->partial_holo, c->W, c->twiH, c->stream); }));
-    return RIHVR_OK;
+    RIHVR_TRY(timed(c, K_ROWS_SUMPARTS, [&] {
+        return c->rad_w ? gen_rows_sumparts(c->W, c->rad_w, est_spec, 1, c->N, c->htmp, c->H, c->twiW, c->stream)
+                        : fft_rows_sumparts(c->W, est_spec, 1, c->N, c->htmp, c->H, c->twiW, c->stream);
+    }));
+    return timed(c, K_COLS_REAL, [&] {
+        return c->rad_h ? gen_cols_real(c->H, c->rad_h, c->htmp, c->hspat, c->meas, c->resid, c->partial_holo, c->W,
+                                        c->twiH, c->stream)
+                        : fft_cols_real(c->H, c->htmp, c->hspat, c->meas, c->resid, c->partial_holo, c->W, c->twiH,
+                                        c->stream);
+    });
 }
 
 rihvr_status apply_forward(rihvr_ctx* c, const float2* vol, float2* est) {
@@ -405,22 +388,14 @@ rihvr_status apply_forward(rihvr_ctx* c, const float2* vol, float2* est) {
 // R-hat = FFT(r) of a spatial residual (SparseGradient::reconstruct, sparse_gradient.cu:47-75)
 // into out; ev_rhat marks rhat
 rihvr_status spectrum(rihvr_ctx* c, const float2* r, float2* out) {
-    if (c->gen) {
-        RIHVR_TRY(timed(c, K_ROWS_PLAIN, [&] { return gen_rows_plain(c->W, -1, r, c->htmp, c->H, c->twfW, c->stream, c->gen_radix); }));
-        RIHVR_TRY(timed(c, K_COLS_PLAIN, [&] {
-            hipError_t e = gen_transpose(c->htmp, c->T2, c->H, c->W, 1, nullptr, false, c->stream);
-            if (e == hipSuccess) e = gen_rows_plain(c->H, -1, c->T2, c->T2, c->W, c->twfH, c->stream, c->gen_radix);
-            if (e == hipSuccess) e = gen_transpose(c->T2, out, c->W, c->H, 1, nullptr, false, c->stream);
-            return e;
-        }));
-        if (out == c->rhat) {
-            c->rhat_scaled = false;
-            RIHVR_HIP(hipEventRecord(c->ev_rhat, c->stream));
-        }
-        return RIHVR_OK;
-    }
-    RIHVR_TRY(timed(c, K_ROWS_PLAIN, [&] { return fft_rows_plain(c->W, -1, r, c->htmp, c->H, c->twfW, c->stream); }));
-    RIHVR_TRY(timed(c, K_COLS_PLAIN, [&] { return fft_cols_plain(c->H, -1, c->htmp, out, c->W, 1, c->twfH, c->stream); }));
+    RIHVR_TRY(timed(c, K_ROWS_PLAIN, [&] {
+        return c->rad_w ? gen_rows_plain(c->W, c->rad_w, -1, r, c->htmp, c->H, c->twfW, c->stream)
+                        : fft_rows_plain(c->W, -1, r, c->htmp, c->H, c->twfW, c->stream);
+    }));
+    RIHVR_TRY(timed(c, K_COLS_PLAIN, [&] {
+        return c->rad_h ? gen_cols_plain(c->H, c->rad_h, -1, c->htmp, out, c->W, 1, c->twfH, c->stream)
+                        : fft_cols_plain(c->H, -1, c->htmp, out, c->W, 1, c->twfH, c->stream);
+    }));
     if (out == c->rhat) {
         c->rhat_scaled = false;
         RIHVR_HIP(hipEventRecord(c->ev_rhat, c->stream));
@@ -440,25 +415,15 @@ rihvr_status rhat_written(rihvr_ctx* c) {
 rihvr_status adjoint_group(rihvr_ctx* c, float2* G, int g0, int gz, hipStream_t st) {
     const float invN = c->rhat_scaled ? 1.0f : (float)(1.0 / (double)c->N);
     float2* Tg = c->T + (size_t)g0 * c->N;
-    if (c->gen) {
-        float2* Tt = c->T2 + (size_t)g0 * c->N;
-        RIHVR_TRY(timed_on(c, K_ROWS_ADJ, st, [&] {
-            return gen_rows_adj(c->W, c->rhat, c->kappa, c->zlist + g0, Tg, c->H, gz, std::min(c->zchunk_adj, gz), invN,
-                                c->twiW, st, c->gen_radix);
-        }));
-        return timed_on(c, K_COLS_ADJ, st, [&] {
-            hipError_t e = gen_transpose(Tg, Tt, c->H, c->W, gz, nullptr, false, st);
-            if (e == hipSuccess) e = gen_rows_plain(c->H, 1, Tt, Tt, (long)gz * c->W, c->twiH, st, c->gen_radix);
-            if (e == hipSuccess) e = gen_transpose(Tt, G + (size_t)g0 * c->N, c->W, c->H, gz, c->phase + g0, false, st);
-            return e;
-        });
-    }
+    const int zc = std::min(c->zchunk_adj, gz);
     RIHVR_TRY(timed_on(c, K_ROWS_ADJ, st, [&] {
-        return fft_rows_adj(c->W, c->rhat, c->kappa, c->zlist + g0, Tg, c->H, gz, std::min(c->zchunk_adj, gz), invN,
-                            c->twiW, st);
+        return c->rad_w ? gen_rows_adj(c->W, c->rad_w, c->rhat, c->kappa, c->zlist + g0, Tg, c->H, gz, zc, invN, c->twiW, st)
+                        : fft_rows_adj(c->W, c->rhat, c->kappa, c->zlist + g0, Tg, c->H, gz, zc, invN, c->twiW, st);
     }));
     RIHVR_TRY(timed_on(c, K_COLS_ADJ, st, [&] {
-        return fft_cols_adj(c->H, Tg, c->phase + g0, G + (size_t)g0 * c->N, c->W, gz, c->twiH, st);
+        float2* Gg = G + (size_t)g0 * c->N;
+        return c->rad_h ? gen_cols_adj(c->H, c->rad_h, Tg, c->phase + g0, Gg, c->W, gz, c->twiH, st)
+                        : fft_cols_adj(c->H, Tg, c->phase + g0, Gg, c->W, gz, c->twiH, st);
     }));
     return RIHVR_OK;
 }
@@ -615,7 +580,7 @@ void release(rihvr_ctx* c) {
     (void)hipFree(c->occ_tmp);
     (void)hipFree(c->occ_ones);
     (void)hipFree(c->smap);
-    void* ptrs[] = {c->G, c->G_alt, c->T, c->T2, c->tvbuf, c->meas, c->hE, c->hC, c->hP, c->hX, c->resid, c->rhat, c->htmp, c->bspec,
+    void* ptrs[] = {c->G, c->G_alt, c->T, c->tvbuf, c->meas, c->hE, c->hC, c->hP, c->hX, c->resid, c->rhat, c->htmp, c->bspec,
                     c->hspat, c->spart, c->kappa,
                     c->zlist, c->phase, c->phase_fwd, c->twfW, c->twiW, c->twfH, c->twiH, c->partial, c->partial_holo, c->scal,
                     c->red_work, c->dflag};
@@ -643,17 +608,28 @@ rihvr_status check_schedule(const rihvr_schedule* s) {
 }
 
 // Planes per workgroup of a row pass that has `blocks` workgroups per plane chunk: as many as
-// leave `target` workgroups, at most `most`, and at least 2 (1 where even single planes do not
-// fill the device).  A workgroup's planes are a serial chain (2.5 us each at L = 256), while more
-// chunks cost A more partial spectra to write and sum.  Forward row pass + spectrum sum, us, by
-// planes per chunk: 256^2 x 32 (16 workgroups a chunk) 2: 22, 8: 31, 32: 86; 512^2 x 100 (128)
-// 4: 75, 16: 62, 32: 87; 448^2 x 40 (112) 8: 40, 32: 83; 1024^2 x 16 (512) 4: 59, 16: 54.  A^T's:
-// 256^2 x 32 1: 11, 2: 12, 8: 25; 512^2 x 20 2: 18, 8: 21; 1024^2 x 16 4: 41, 8: 37.
-int split_planes(int nz, int blocks, int target, int most) {
+// leave `target` workgroups, at most `most`, and at least 2 (4 where that still leaves 768 workgroups
+// of the run-time plans; 1 where even single planes do not fill the device).  A workgroup's planes
+// are a serial chain (2.5 us each at L = 256), while more chunks cost A more partial spectra to write
+// and sum, and every workgroup its tables.  Forward row pass + spectrum sum, us, by planes per
+// chunk: 256^2 x 32 (16 workgroups a chunk) 2: 22, 8: 31, 32: 86; 512^2 x 100 (128) 4: 75, 16: 62,
+// 32: 87; 448^2 x 40 (112) 8: 40, 32: 83; 1024^2 x 16 (512) 4: 59, 16: 54.  A^T's: 256^2 x 32 1: 11,
+// 2: 12, 8: 25; 512^2 x 20 2: 18, 8: 21; 1024^2 x 16 4: 41, 8: 37.  Run-time plans, forward: 1280 x
+// 1024 x 40 8: 243, 20: 471; A^T: 1040 x 464 x 24 2: 97, 4: 62.
+int split_planes(int nz, int blocks, bool run_time, int target, int most) {
     const int chunks = (target + blocks - 1) / blocks;
     const int zc = (nz + chunks - 1) / chunks;
-    const int least = (long)nz * blocks <= 256 ? 1 : 2;
+    const long all = (long)nz * blocks;
+    const int least = all <= 256 ? 1 : run_time && all >= 4 * 768 ? 4 : 2;
     return std::max(std::min(zc, most), least);
+}
+
+// the plane chunks of A's and A^T's row passes without a schedule
+void default_chunks(int W, int H, int nz, int* fwd, int* adj) {
+    const bool fixed = fft_length_supported(W);
+    const int blocks = fixed ? fft_rows_blocks(W, H) : gen_rows_blocks(W, H);
+    *fwd = split_planes(nz, blocks, !fixed, fixed ? 640 : 2560, 32);
+    *adj = split_planes(nz, blocks, !fixed, fixed ? 1024 : 2560, 8);
 }
 
 // sch: the launch choices (NULL: the defaults, with the RIHVR_* environment overrides)
@@ -686,10 +662,7 @@ rihvr_status create_impl(const rihvr_params* params, const rihvr_schedule* sch, 
         force_gen = sch->fft_path == 1;
         c->graphs = sch->graphs != 0;
     } else {
-        if (fft_length_supported(c->W) && fft_length_supported(c->H)) {
-            zc = split_planes(c->Nz, fft_rows_blocks(c->W, c->H), 640, 32);
-            za = split_planes(c->Nz, fft_rows_blocks(c->W, c->H), 1024, 8);
-        }
+        default_chunks(c->W, c->H, c->Nz, &zc, &za);
         if (const char* e = std::getenv("RIHVR_ZCHUNK")) zc = std::max(1, std::atoi(e));
         if (const char* e = std::getenv("RIHVR_ZCHUNK_ADJ")) za = std::max(1, std::atoi(e));
         if (const char* e = std::getenv("RIHVR_PROX_ROWS")) prow = std::max(0, std::atoi(e));
@@ -711,10 +684,11 @@ rihvr_status create_impl(const rihvr_params* params, const rihvr_schedule* sch, 
     pp = ((pp + 15) / 16) * 16;
     c->pipe_planes = std::min(c->Nz, std::max(16, pp));
     if (c->pipe_planes % c->zchunk_fwd || c->pipe_planes % c->zchunk_adj) c->pipe_planes = c->Nz;
-    c->gen = force_gen || !(fft_length_supported(c->W) && fft_length_supported(c->H));
+    c->rad_w = force_gen || !fft_length_supported(c->W) ? c->gen_radix : 0;
+    c->rad_h = force_gen || !fft_length_supported(c->H) ? c->gen_radix : 0;
     const bool tv_general = params->mode == RIHVR_MODE_FASTA_FUSED_LASSO_2D &&
                             !prox_fl2d_supported(params->num_tv_iterations);
-    if (c->gen || tv_general) c->pipe_planes = c->Nz;  // the plane-group schedule needs the fused kernels
+    if (tv_general) c->pipe_planes = c->Nz;  // the plane-group schedule needs the fused prox
     c->n_groups = (c->Nz + c->pipe_planes - 1) / c->pipe_planes;
     if (const char* e = std::getenv("RIHVR_GROUP_ONE_STREAM")) c->groups_one_stream = std::atoi(e) != 0;
     if (const char* e = std::getenv("RIHVR_TEST_BACKTRACKS")) c->test_backtracks = std::strtoull(e, nullptr, 0);
@@ -729,7 +703,6 @@ rihvr_status create_impl(const rihvr_params* params, const rihvr_schedule* sch, 
     RIHVR_TRY(dalloc(&c->G, c->V));
     RIHVR_TRY(dalloc(&c->G_alt, c->V));
     RIHVR_TRY(dalloc(&c->T, c->V));
-    if (c->gen) RIHVR_TRY(dalloc(&c->T2, c->V));
     if (tv_general) RIHVR_TRY(dalloc(&c->tvbuf, 4 * (size_t)c->V));
     float2** holos[] = {&c->meas, &c->hE, &c->hC, &c->hP, &c->hX, &c->resid, &c->rhat, &c->htmp, &c->bspec, &c->hspat};
     for (float2** h : holos) RIHVR_TRY(dalloc(h, c->N));
@@ -758,7 +731,7 @@ rihvr_status create_impl(const rihvr_params* params, const rihvr_schedule* sch, 
     c->partial_rows = rows;
     RIHVR_TRY(dalloc(&c->partial, (size_t)rows * PS_COUNT));
     c->holo_rows = std::max<long>(std::max<long>(holo_num_blocks(c->N), c->W / 16), holo_spec_num_blocks(c->W, c->H));
-    c->holo_rows = std::max<long>(c->holo_rows, gen_transpose_real_blocks(c->H, c->W));
+    if (c->rad_h) c->holo_rows = std::max<long>(c->holo_rows, gen_cols_blocks(c->H, c->W));
     RIHVR_TRY(dalloc(&c->partial_holo, c->holo_rows));
     RIHVR_TRY(dalloc(&c->scal, SL_COUNT));
     RIHVR_TRY(dalloc(&c->red_work, (size_t)kReduceBlocks * PS_COUNT));
@@ -1451,7 +1424,7 @@ rihvr_status lipschitz_impl(rihvr_ctx* c, int seed, int iterations, double* L) {
 
 rihvr_schedule schedule_of(const rihvr_ctx* c) {
     rihvr_schedule s{};
-    s.fft_path = c->gen ? 1 : 0;
+    s.fft_path = c->rad_w || c->rad_h ? 1 : 0;
     s.max_radix = c->gen_radix;
     s.zchunk_fwd = c->zchunk_fwd;
     s.zchunk_adj = c->zchunk_adj;
@@ -1532,8 +1505,7 @@ rihvr_status autotune_impl(const rihvr_params* p, const float* holo, int holo_lo
     // the starting point: the defaults
     rihvr_schedule cur{};
     cur.max_radix = 16;
-    cur.zchunk_fwd = std::min(32, p->num_planes);
-    cur.zchunk_adj = std::min(8, p->num_planes);
+    default_chunks(p->width, p->height, p->num_planes, &cur.zchunk_fwd, &cur.zchunk_adj);
     cur.graphs = 1;
     const bool fixed = fft_length_supported(p->width) && fft_length_supported(p->height);
     if (!fixed) cur.fft_path = 1;
@@ -1560,14 +1532,14 @@ rihvr_status autotune_impl(const rihvr_params* p, const float* holo, int holo_lo
     RIHVR_TRY(try_set(v));
     const rihvr_schedule base = cur;
     v.clear();
-    for (int z : {8, 16, 32, 64}) {
+    for (int z : {2, 4, 8, 16, 32, 64}) {
         rihvr_schedule s = base;
         s.zchunk_fwd = std::min(z, p->num_planes);
         v.push_back(s);
     }
     RIHVR_TRY(try_set(v));
     v.clear();
-    for (int z : {4, 8, 16, 32}) {
+    for (int z : {2, 4, 8, 16, 32}) {
         rihvr_schedule s = cur;
         s.zchunk_adj = std::min(z, p->num_planes);
         v.push_back(s);
