@@ -179,8 +179,8 @@ hipError_t soft_threshold_map2(const float2* in, int W, int H, int nz, float tau
 hipError_t norm2_partials(const float2* v, long n, int nblocks, double* partial, hipStream_t s);
 // a sparse pseudo-random volume (about 1 / period of its voxels non-zero)
 hipError_t synth_volume(float2* v, long n, unsigned period, unsigned seed, hipStream_t s);
-// *f = fv and *d = dv (either may be NULL), in stream order
-hipError_t set_scalars(float* f, float fv, double* d, double dv, hipStream_t s);
+// *f = fv, *d = dv and map[0 .. n) = 0 (n may be 0), in stream order
+hipError_t begin_iteration(float* f, float fv, double* d, double dv, uint64_t* map, long n, hipStream_t s);
 // resid = est - meas with partial sum |resid|^2
 hipError_t holo_residual(const float2* est, const float2* meas, float2* resid, long n, double* partial,
                          hipStream_t s);
@@ -194,9 +194,11 @@ hipError_t holo_spec(const float2* parts, int nparts, long stride, int W, int H,
 hipError_t holo_scale(const float2* in, float2* out, long n, float f, hipStream_t s);
 
 // sums rows of partial [nrows][ncols] into out[ncols] (fixed order: deterministic);
-// work holds kReduceBlocks * ncols doubles
+// work holds kReduceBlocks * ncols doubles.  Then pub_dst[0 .. pub_n) = pub_src[0 .. pub_n), when
+// set (pinned host memory; it may include out).
 constexpr int kReduceBlocks = 64;
-hipError_t reduce_partials(const double* partial, int nrows, int ncols, double* work, double* out, hipStream_t s);
+hipError_t reduce_partials(const double* partial, int nrows, int ncols, double* work, double* out, hipStream_t s,
+                           const double* pub_src = nullptr, double* pub_dst = nullptr, int pub_n = 0);
 
 // flags[0] = 1 if any element of a [n] complex array is not finite
 hipError_t check_finite(const float2* a, long n, int* flag, hipStream_t s);

@@ -1410,12 +1410,17 @@ hipError_t synth_volume(float2* v, long n, unsigned period, unsigned seed, hipSt
     return hipGetLastError();
 }
 
-__global__ void k_set_scalars(float* __restrict__ f, float fv, double* __restrict__ d, double dv) {
-    if (f) *f = fv;
-    if (d) *d = dv;
+__global__ void k_begin_iteration(float* f, float fv, double* d, double dv, uint64_t* __restrict__ map, long n) {
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) {
+        *f = fv;
+        *d = dv;
+    }
+    if (i < n) map[i] = 0ull;
 }
-hipError_t set_scalars(float* f, float fv, double* d, double dv, hipStream_t s) {
-    hipLaunchKernelGGL(k_set_scalars, dim3(1), dim3(1), 0, s, f, fv, d, dv);
+hipError_t begin_iteration(float* f, float fv, double* d, double dv, uint64_t* map, long n, hipStream_t s) {
+    hipLaunchKernelGGL(k_begin_iteration, dim3((unsigned)std::max(1L, (n + 255) / 256)), dim3(256), 0, s, f, fv, d, dv,
+                       map, n);
     return hipGetLastError();
 }
 
@@ -1596,9 +1601,8 @@ hipError_t holo_scale(const float2* in, float2* out, long n, float f, hipStream_
     return hipGetLastError();
 }
 
-// Two fixed-order passes (deterministic): kReduceBlocks workgroups each sum a
-// contiguous slice of rows of every column (row-contiguous, coalesced loads) into
-// work[block][ncols]; one workgroup then sums those rows in block order.
+// First pass over many rows (deterministic): kReduceBlocks workgroups each sum a contiguous slice
+// of rows of every column (row-contiguous, coalesced loads) into work[block][ncols].
 constexpr int kReduceThreads = 256;
 __global__ void __launch_bounds__(kReduceThreads) k_reduce_rows(const double* __restrict__ partial, int nrows,
                                                                 int ncols, int rows_per_block, double* out) {
@@ -1622,15 +1626,59 @@ __global__ void __launch_bounds__(kReduceThreads) k_reduce_rows(const double* __
     }
 }
 
-hipError_t reduce_partials(const double* partial, int nrows, int ncols, double* work, double* out, hipStream_t s) {
-    if (ncols < 1 || ncols > PS_COUNT || nrows < 0) return hipErrorInvalidValue;
-    const int rpb = (nrows + kReduceBlocks - 1) / kReduceBlocks;
-    const int nb = rpb > 0 ? (nrows + rpb - 1) / rpb : 1;
-    hipLaunchKernelGGL(k_reduce_rows, dim3(nb), dim3(kReduceThreads), 0, s, partial, nrows, ncols, rpb > 0 ? rpb : 1,
-                       work);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_reduce_rows, dim3(1), dim3(kReduceThreads), 0, s, (const double*)work, nb, ncols, nb, out);
+// The sums of all columns by one workgroup, in a fixed order; then pub_dst[0 .. pub_n) = pub_src
+// (host memory that the device writes: the scalars reach the host with the sums, without a copy).
+constexpr int kReduceOneThreads = 1024;
+__global__ void __launch_bounds__(kReduceOneThreads)
+k_reduce_one(const double* __restrict__ partial, int nrows, int ncols, double* out, const double* pub_src,
+             double* pub_dst, int pub_n) {
+    __shared__ double red[PS_COUNT][kReduceOneThreads / 64];
+    double acc[PS_COUNT];
+#pragma unroll
+    for (int q = 0; q < PS_COUNT; ++q) acc[q] = 0.0;
+    for (int r = threadIdx.x; r < nrows; r += kReduceOneThreads) {
+        const double* row = partial + (size_t)r * ncols;
+#pragma unroll
+        for (int q = 0; q < PS_COUNT; ++q)
+            if (q < ncols) acc[q] += row[q];
+    }
+#pragma unroll
+    for (int q = 0; q < PS_COUNT; ++q) {
+        if (q >= ncols) break;
+        const double v = wave_sum(acc[q]);
+        if ((threadIdx.x & 63) == 0) red[q][threadIdx.x >> 6] = v;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < ncols) {
+        double r = 0.0;
+        for (int w = 0; w < kReduceOneThreads / 64; ++w) r += red[threadIdx.x][w];
+        out[threadIdx.x] = r;
+    }
+    if (!pub_dst) return;
+    __threadfence();
+    __syncthreads();
+    if ((int)threadIdx.x < pub_n) pub_dst[threadIdx.x] = pub_src[threadIdx.x];
+}
+
+// One workgroup takes up to this many rows by itself: a launch less, which is what a reduction
+// costs at small sizes (256^2 x 32: 5 us each); at 12,160 rows of 8 two launches take 10 us and one
+// workgroup would read 0.8 MB alone.
+constexpr int kReduceOneRows = 4096;
+
+hipError_t reduce_partials(const double* partial, int nrows, int ncols, double* work, double* out, hipStream_t s,
+                           const double* pub_src, double* pub_dst, int pub_n) {
+    if (ncols < 1 || ncols > PS_COUNT || nrows < 0 || pub_n > kReduceOneThreads) return hipErrorInvalidValue;
+    if (nrows > kReduceOneRows) {
+        const int rpb = (nrows + kReduceBlocks - 1) / kReduceBlocks;
+        const int nb = (nrows + rpb - 1) / rpb;
+        hipLaunchKernelGGL(k_reduce_rows, dim3(nb), dim3(kReduceThreads), 0, s, partial, nrows, ncols, rpb, work);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        partial = work;
+        nrows = nb;
+    }
+    hipLaunchKernelGGL(k_reduce_one, dim3(1), dim3(kReduceOneThreads), 0, s, partial, nrows, ncols, out, pub_src,
+                       pub_dst, pub_n);
     return hipGetLastError();
 }
 

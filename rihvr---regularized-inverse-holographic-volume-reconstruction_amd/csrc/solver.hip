@@ -35,7 +35,7 @@ constexpr double kPi = 3.14159265358979323846;
 constexpr double kDenseFraction = 0.05;
 
 // scalar slots after reduction
-enum Slot { SL_PROX = 0, SL_RESID_A = 8, SL_RESID_M = 9, SL_COUNT = 16 };
+enum Slot { SL_PROX = 0, SL_RESID_A = 8, SL_RESID_M = 9, SL_FLAG = 10, SL_COUNT = 16 };
 
 #define RIHVR_HIP(call)                                                   \
     do {                                                                  \
@@ -291,12 +291,9 @@ rihvr_status fetch_scalars(rihvr_ctx* c) {
     return resolve_timing(c);
 }
 
-// The same copy, waited for by an event so that work queued after it keeps the device busy.
-rihvr_status fetch_scalars_async(rihvr_ctx* c) {
-    RIHVR_HIP(hipMemcpyAsync(c->h_scal, c->scal, SL_COUNT * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    RIHVR_HIP(hipEventRecord(c->ev_scal, c->stream));
-    return RIHVR_OK;
-}
+// The scalars as A's reduction (forward_finish) wrote them to h_scal, waited for by an event
+// recorded after it, so that work queued later keeps the device busy.  The next A writes h_scal
+// again: it is queued only after the host has read it.
 rihvr_status wait_scalars(rihvr_ctx* c) {
     RIHVR_HIP(hipEventSynchronize(c->ev_scal));
     scale_resid_norms(c);
@@ -358,7 +355,7 @@ rihvr_status forward_finish(rihvr_ctx* c, float2* est) {
     }));
     RIHVR_TRY(timed(c, K_REDUCE, [&] {
         return reduce_partials(c->partial_holo, holo_spec_num_blocks(c->W, c->H), 1, c->red_work, c->scal + SL_RESID_A,
-                               c->stream);
+                               c->stream, c->scal, c->h_scal, SL_COUNT);
     }));
     return RIHVR_OK;
 }
@@ -445,7 +442,8 @@ int effective_mode(const rihvr_ctx* c) {
 bool tv3d(const rihvr_ctx* c) { return c->ss.mode == RIHVR_MODE_FASTA_FUSED_LASSO; }
 
 // y = prox(x0 - t g), x0 = Y0 + s (Y0 - YM); reductions into scal[SL_PROX..]
-// s_mom_dev (may be NULL): the momentum step in device memory (a captured graph reads it there);
+// s_mom_dev (may be NULL): the momentum step in device memory (a captured graph reads it there),
+// set by begin_iteration, which also cleared the map;
 // enqueue = false performs only the host-side bookkeeping of the maps (a replayed graph holds
 // the launches)
 rihvr_status apply_prox(rihvr_ctx* c, int mode, const float2* Y0, const float2* YM, float s_mom, const float2* G,
@@ -484,7 +482,8 @@ rihvr_status apply_prox(rihvr_ctx* c, int mode, const float2* Y0, const float2* 
         a.occ_new = c->occ_tmp;
         a.occ_new_planes = c->occ_tmp + (size_t)c->Nz * c->H;
         if (enqueue) {
-            RIHVR_HIP(fill_u64(c->occ_tmp, (long)map_words(c), 0ull, c->stream));
+            // (with s_mom_dev the map is cleared by the launch that set it)
+            if (!s_mom_dev) RIHVR_HIP(fill_u64(c->occ_tmp, (long)map_words(c), 0ull, c->stream));
             RIHVR_TRY(timed(c, K_PROX, [&] { return prox_fl2d(a, c->stream); }));
         }
         rows = prox_fl2d_num_waves(c->W, c->H, c->Nz, a.n_tv, c->prox_rows);
@@ -793,12 +792,9 @@ rihvr_status begin_impl(rihvr_ctx* c, const float* holo, int holo_loc, const flo
     c->ss = SolveState{};
     c->ss.mode = effective_mode(c);
     RIHVR_TRY(copy_in(c, c->meas, holo, holo_loc, c->N));
-    RIHVR_HIP(hipMemsetAsync(c->dflag, 0, sizeof(int), c->stream));
-    RIHVR_HIP(check_finite(c->meas, c->N, c->dflag, c->stream));
-    int hflag = 0;
-    RIHVR_HIP(hipMemcpyAsync(&hflag, c->dflag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    RIHVR_HIP(hipStreamSynchronize(c->stream));
-    if (hflag) return RIHVR_E_INVALID_DATA;
+    // a non-finite value is found with the initial residual's scalars, below
+    RIHVR_HIP(hipMemsetAsync(c->scal + SL_FLAG, 0, sizeof(double), c->stream));
+    RIHVR_HIP(check_finite(c->meas, c->N, (int*)(c->scal + SL_FLAG), c->stream));
     // the measurement's spectrum FFT(b) / N
     RIHVR_TRY(spectrum(c, c->meas, c->bspec));
     RIHVR_HIP(holo_scale(c->bspec, c->bspec, c->N, (float)(1.0 / (double)c->N), c->stream));
@@ -831,7 +827,10 @@ rihvr_status begin_impl(rihvr_ctx* c, const float* holo, int holo_loc, const flo
         // slots of a warm start with a map (the learned start) hold the network's output and
         // the threshold candidates, and no candidate is chosen when they hold a NaN.
     } else {
-        RIHVR_HIP(hipMemcpyAsync(YM, Y0, c->V * sizeof(float2), hipMemcpyDeviceToDevice, c->stream));
+        if (warm)
+            RIHVR_HIP(hipMemcpyAsync(YM, Y0, c->V * sizeof(float2), hipMemcpyDeviceToDevice, c->stream));
+        else
+            RIHVR_HIP(hipMemsetAsync(YM, 0, c->V * sizeof(float2), c->stream));
         if (keep_map) {
             RIHVR_HIP(hipMemcpyAsync(c->occ[c->iym], c->occ[in_ring], map_words(c) * sizeof(uint64_t),
                                      hipMemcpyDeviceToDevice, c->stream));
@@ -861,6 +860,9 @@ rihvr_status begin_impl(rihvr_ctx* c, const float* holo, int holo_loc, const flo
         }));
     }
     RIHVR_TRY(fetch_scalars(c));
+    int hflag = 0;
+    std::memcpy(&hflag, c->h_scal + SL_FLAG, sizeof(int));
+    if (hflag) return RIHVR_E_INVALID_DATA;
     if (warm) {
         l1 = c->h_scal[SL_PROX + PS_L1X0];
         tv = c->h_scal[SL_PROX + PS_TVX0];
@@ -965,6 +967,7 @@ rihvr_status iterate_impl(rihvr_ctx* c, int n_it, rihvr_stats* st, bool last_f_b
         float2* Y0 = c->Yb[c->iy0];
         float2* YM = c->Yb[c->iym];
         bool queued = false;  // the accepted-iteration work is queued
+        const double a1 = (1.0 + std::sqrt(1.0 + 4.0 * alpha0 * alpha0)) / 2.0;  // alpha_{k+1} without a restart
         const bool dense = c->dense_ok && s.nnz_y >= kDenseFraction * (double)c->V;
         for (;;) {
             const bool use_graph = ahead && c->graphs && !c->tm.on;
@@ -975,7 +978,10 @@ rihvr_status iterate_impl(rihvr_ctx* c, int n_it, rihvr_stats* st, bool last_f_b
                     for (int g0 = 0; g0 < c->Nz; g0 += c->pipe_planes)
                         RIHVR_TRY(adjoint_group(c, c->G, g0, std::min(c->pipe_planes, c->Nz - g0), c->stream));
                 if (use_graph) {
-                    RIHVR_HIP(set_scalars(c->d_smom, s.s_mom, nullptr, 0.0, c->stream));
+                    // the steps that the replayed graphs read, and the map that the prox builds
+                    const bool maps = mode == RIHVR_MODE_FASTA_FUSED_LASSO_2D && !c->tvbuf && !dense;
+                    RIHVR_HIP(begin_iteration(c->d_smom, s.s_mom, c->d_step, (alpha0 - 1) / a1, c->occ_tmp,
+                                              maps ? (long)map_words(c) : 0L, c->stream));
                     const std::vector<const void*> key = {
                         Y0, YM, Yn, c->G, c->hX, c->occ[0], c->occ[1], c->occ[2], c->occ_tmp,
                         (const void*)(intptr_t)(c->occ_valid[0] | (c->occ_valid[1] << 1) | (c->occ_valid[2] << 2)),
@@ -994,12 +1000,10 @@ rihvr_status iterate_impl(rihvr_ctx* c, int n_it, rihvr_stats* st, bool last_f_b
             }
             s.g_ready = true;
             if (ahead) {
-                RIHVR_TRY(fetch_scalars_async(c));
-                const double a1 = (1.0 + std::sqrt(1.0 + 4.0 * alpha0 * alpha0)) / 2.0;
+                RIHVR_HIP(hipEventRecord(c->ev_scal, c->stream));
                 std::swap(c->hP, c->hC);
                 std::swap(c->hC, c->hX);
                 if (use_graph) {
-                    RIHVR_HIP(set_scalars(nullptr, 0.0f, c->d_step, (alpha0 - 1) / a1, c->stream));
                     c->rhat_scaled = true;  // the graph's hologram momentum writes the residual spectrum
                     const bool next = i + 1 < n_it;
                     const std::vector<const void*> key = {c->hC, c->hP, c->hE, c->rhat, c->G_alt,
