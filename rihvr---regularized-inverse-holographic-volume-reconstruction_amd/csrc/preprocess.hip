@@ -80,8 +80,12 @@ struct Geometry {
     int rw, rh, pad, ow, oh;
 };
 
-// output pixels PIX * (blockIdx.x * kThreads + threadIdx.x) + [0, PIX) of row blockIdx.y of frame
-// blockIdx.z + f0; PIX = kPix needs ow % kPix == 0 and a 16-byte aligned output (two complex per store).
+// Output pixels of row blockIdx.y of frame blockIdx.z + f0: one per thread (PIX = 1), or PIX / 2 pairs
+// per thread, 2 kThreads pixels apart, so that every 16-byte store (two complex) of a wave is
+// contiguous; that needs an even ow and a 16-byte aligned output.  The holograms are written past
+// the caches: they are eight times the frames' bytes and read by a later call.  What bounds it is that
+// stream: 100 frames of 1024^2 take 183 us a call (5.2 TB/s, a copy reaches 5.14), 281 before with 32 bytes a
+// thread in two ordinary stores.
 // Every pixel's loads are issued unconditionally (pixel 0 of the frame stands in for a pixel outside
 // the crop or the image) so that they overlap; the select afterwards keeps zero for those pixels.
 template <typename T, int PIX>
@@ -91,8 +95,9 @@ __global__ void __launch_bounds__(kThreads) k_pre_write(const T* __restrict__ fr
                                                         const float* __restrict__ inv_mean,
                                                         float2* __restrict__ out) {
 #pragma clang fp contract(off)  // the host function's separate float roundings
-    const int x = PIX * (blockIdx.x * kThreads + threadIdx.x);
-    if (x >= g.ow) return;
+    const int x0 = PIX == 1 ? blockIdx.x * kThreads + threadIdx.x : PIX * blockIdx.x * kThreads + 2 * threadIdx.x;
+    if (x0 >= g.ow) return;
+    auto px = [&](int k) { return PIX == 1 ? x0 : x0 + (k >> 1) * 2 * kThreads + (k & 1); };  // pixel k's column
     const int y = blockIdx.y;
     const int f = f0 + blockIdx.z;
     const T* fr = frames + (size_t)f * g.W * g.H;
@@ -102,7 +107,7 @@ __global__ void __launch_bounds__(kThreads) k_pre_write(const T* __restrict__ fr
     long si[PIX];
 #pragma unroll
     for (int k = 0; k < PIX; ++k) {
-        const int cx = x + k - g.pad, sx = g.src_x0 + cx;
+        const int cx = px(k) - g.pad, sx = g.src_x0 + cx;
         in[k] = row_in && cx >= 0 && cx < g.rw && sx >= 0 && sx < g.W;
         si[k] = in[k] ? (long)sy * g.W + sx : 0;
     }
@@ -125,12 +130,14 @@ __global__ void __launch_bounds__(kThreads) k_pre_write(const T* __restrict__ fr
 #pragma unroll
         for (int k = 0; k < PIX; ++k) v[k] = in[k] ? h[k] * im - 1.0f : 0.0f;
     }
-    float2* o = out + ((size_t)f * g.oh + y) * g.ow + x;
+    float2* o = out + ((size_t)f * g.oh + y) * g.ow;
     if constexpr (PIX == 1) {
-        *o = make_float2(v[0], 0.0f);
+        o[x0] = make_float2(v[0], 0.0f);
     } else {
+        typedef float f4 __attribute__((ext_vector_type(4)));
 #pragma unroll
-        for (int k = 0; k < PIX; k += 2) ((float4*)o)[k / 2] = make_float4(v[k], 0.0f, v[k + 1], 0.0f);
+        for (int k = 0; k < PIX; k += 2)
+            if (px(k) < g.ow) __builtin_nontemporal_store(f4{v[k], 0.0f, v[k + 1], 0.0f}, (f4*)(o + px(k)));
     }
 }
 
@@ -174,7 +181,7 @@ rihvr_status run_with(const T* frames, const float* bg, const Geometry& g, int n
         PRE_HIP(hipGetLastError());
     }
     // frames in launches of at most kMaxGridYZ (the grid's y and z limit)
-    const bool wide = g.ow % kPix == 0 && (size_t)out_dev % 16 == 0;
+    const bool wide = g.ow % 2 == 0 && (size_t)out_dev % 16 == 0;
     const int pix = wide ? kPix : 1;
     for (int f0 = 0; f0 < n; f0 += kMaxGridYZ) {
         const dim3 grid((unsigned)((g.ow + kThreads * pix - 1) / (kThreads * pix)), (unsigned)g.oh,
