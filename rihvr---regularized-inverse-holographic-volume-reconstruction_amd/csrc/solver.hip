@@ -231,6 +231,18 @@ rihvr_status copy_out(rihvr_ctx* c, float* dst, const float2* src, int loc, size
     return RIHVR_OK;
 }
 
+// Whether the context's kernels can work on caller memory in place: device memory of its GPU,
+// aligned for complex64.  Anything else that a copy accepts is copied.
+bool in_place(const rihvr_ctx* c, const void* p, int loc) {
+    if (loc != RIHVR_DEVICE || (uintptr_t)p % sizeof(float2)) return false;
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type == hipMemoryTypeDevice && a.device == c->device;
+}
+
 // Launches through `launch` (returns hipError_t) on stream `st`, bracketed by events
 // on that stream when timing is on.
 template <class F> rihvr_status timed_on(rihvr_ctx* c, int id, hipStream_t st, F&& launch) {
@@ -1808,9 +1820,12 @@ rihvr_status rihvr_forward(rihvr_ctx* ctx, const float* volume, int vol_loc, flo
     if (!ctx || !volume || !holo_out) return RIHVR_E_INVALID_ARGUMENT;
     ctx->have_result = false;
     ctx->ss.active = false;
-    float2* v = ctx->Yb[0];
-    ctx->occ_valid[0] = false;
-    RIHVR_TRY(copy_in(ctx, v, volume, vol_loc, ctx->V));
+    const float2* v = (const float2*)volume;
+    if (!in_place(ctx, volume, vol_loc)) {
+        ctx->occ_valid[0] = false;
+        RIHVR_TRY(copy_in(ctx, ctx->Yb[0], volume, vol_loc, ctx->V));
+        v = ctx->Yb[0];
+    }
     RIHVR_HIP(hipMemsetAsync(ctx->meas, 0, ctx->N * sizeof(float2), ctx->stream));
     RIHVR_HIP(hipMemsetAsync(ctx->bspec, 0, ctx->N * sizeof(float2), ctx->stream));
     RIHVR_TRY(apply_forward(ctx, v, ctx->hE));
@@ -1823,6 +1838,13 @@ rihvr_status rihvr_adjoint(rihvr_ctx* ctx, const float* holo, int holo_loc, floa
     ctx->have_result = false;
     ctx->ss.active = false;
     RIHVR_TRY(copy_in(ctx, ctx->resid, holo, holo_loc, ctx->N));
+    // the last pass writes a device volume where the caller wants it (the copy was 210 of 830 us at
+    // 2048^2 x 16)
+    if (in_place(ctx, volume_out, vol_loc)) {
+        RIHVR_TRY(apply_adjoint(ctx, ctx->resid, (float2*)volume_out));
+        RIHVR_HIP(hipStreamSynchronize(ctx->stream));
+        return RIHVR_OK;
+    }
     RIHVR_TRY(apply_adjoint(ctx, ctx->resid, ctx->G));
     return copy_out(ctx, volume_out, ctx->G, vol_loc, ctx->V);
 }
