@@ -364,6 +364,7 @@ struct GenRowArgs {
     const float2* tw;     // W_L^m for the transform's sign
     int nrows;            // rows per plane (ADJ, FWDACC) or in total (PLAIN, SUMPART)
     const float2* rhat;   // ADJ: [nrows][L]
+    bool stream_out;      // ADJ: the output is larger than the caches
     const double* kappa;  // ADJ, FWDACC: [nrows][L]
     const float* zlist;
     int nz, zchunk;
@@ -374,10 +375,6 @@ struct GenRowArgs {
 };
 
 inline int row_pitch(int L) { return L + L / 16 + 1; }
-
-// Hides v's value from the compiler.  In a loop over planes every pass's indices are the same for
-// each plane, and it would keep those of all radices in registers across the loop (184 VGPRs).
-__device__ __forceinline__ void fresh(int& v) { asm volatile("" : "+v"(v)); }
 
 template <int SIGN, int MODE>
 __global__ void __launch_bounds__(kRowMaxThreads, 5) k_gen_rows(GenRowArgs a) {
@@ -427,7 +424,7 @@ __global__ void __launch_bounds__(kRowMaxThreads, 5) k_gen_rows(GenRowArgs a) {
             run_plan<SIGN>(
                 a.plan, map, buf, tw, true,
                 [&](int s, int, int) { return cscale(cmul(transfer(zz, kp[s]), rh[s]), a.invN); }, 0,
-                [&](int w, int j, float2 v) { dst[w * L + j] = v; });
+                [&](int w, int j, float2 v) { store_stream(dst + (w * L + j), v, a.stream_out); });
         }
     } else {  // GR_FWDACC: forward FFT along x, times H_{-z}, summed over a chunk of planes
         // the transform's results stay in LDS and are taken from there in raster order, so that a
@@ -567,11 +564,13 @@ template <int SIGN, int MODE> __global__ void __launch_bounds__(1024) k_gen_cols
         float2* dst = a.out + (size_t)z * L * W + col0;
         float2 ph = make_float2(1.0f, 0.0f);
         if constexpr (MODE == GC_ADJ) ph = a.phase[z];
+        const bool wide = a.sh >= 4;  // whole memory lines (narrower strips share them through the caches)
         run_plan<SIGN>(
-            a.plan, map, buf, tw, true, [&](int, int w, int j) { return src[(size_t)j * W + w]; }, 0,
+            a.plan, map, buf, tw, true,
+            [&](int, int w, int j) { return load_stream(src + ((size_t)j * W + w), MODE == GC_ADJ && wide); }, 0,
             [&](int w, int j, float2 v) {
                 if constexpr (MODE == GC_ADJ) v = make_float2(v.x * ph.x - v.y * ph.y, v.y * ph.x + v.x * ph.y);
-                dst[(size_t)j * W + w] = v;
+                store_stream(dst + ((size_t)j * W + w), v, MODE == GC_ADJ && wide);
             });
     } else if constexpr (MODE == GC_FWD) {
         const float2 ph = a.phase[z];
@@ -660,6 +659,7 @@ hipError_t gen_rows_adj(int L, int radix, const float2* rhat, const double* kapp
     GenRowArgs a{};
     a.out = out; a.tw = tw_inv; a.nrows = nrows; a.rhat = rhat; a.kappa = kappa; a.zlist = zlist; a.nz = nz;
     a.zchunk = zchunk; a.invN = invN;
+    a.stream_out = streams(L, nrows, nz);
     return launch_rows<1, GR_ADJ>(a, L, radix, (unsigned)((nz + zchunk - 1) / zchunk), s);
 }
 

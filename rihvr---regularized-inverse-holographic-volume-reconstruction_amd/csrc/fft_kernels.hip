@@ -52,6 +52,7 @@ struct RowArgs {
     const float2* twg;      // W_L^m table for the transform sign
     // ADJ
     const float2* rhat;     // [H][L] spectrum of the residual
+    bool stream_out;        // the output is larger than the caches (streams())
     const double* kappa;    // [H][L]
     const float* zlist;     // plane positions
     int nz, zchunk;
@@ -69,6 +70,11 @@ struct RowArgs {
 // other lengths, whose plans hold more elements per thread, the extra registers cost waves per
 // SIMD (576, 768, 832: 2 -> 1), so those keep the plain passes.
 template <int L> constexpr bool row_regs_fast() { return L == 1024; }
+// Above 512 (and below 1024) the passes' indices are computed for each plane anew: kept across the
+// planes they cost waves per SIMD (forward pass at 896^2 x 32 138 -> 79 us, 640^2 x 64 94 -> 81,
+// 576^2 x 64 94 -> 79; at 512^2 x 100, where the registers allow it, keeping them is faster, 61
+// against 68 us).
+template <int L> constexpr bool row_fresh() { return L > 512; }
 
 template <int L, int SIGN, int MODE>
 __global__ void __launch_bounds__(RowCfg<L>::THREADS) k_rows(RowArgs a) {
@@ -140,8 +146,10 @@ __global__ void __launch_bounds__(RowCfg<L>::THREADS) k_rows(RowArgs a) {
                 if (!smask) continue;
                 const double mz = -(double)a.zlist[z];
                 const float2* src_row = a.in + ((size_t)z * a.nrows + rrow) * L;
+                int tz = t;
+                if constexpr (row_fresh<L>()) fresh(tz);
                 FftRun<L, SIGN, typename Plan::radices, Plan::TPT>::run(
-                    tw_s, t,
+                    tw_s, tz,
                     [&](int, int, int j) {
                         return ((smask >> (j >> 4)) & 1ull) ? src_row[j] : make_float2(0.0f, 0.0f);
                     },
@@ -237,7 +245,7 @@ __global__ void __launch_bounds__(RowCfg<L>::THREADS) k_rows(RowArgs a) {
                     float2 h = transfer(zz, kp[i][r]);
                     return cscale(cmul(h, rh[i][r]), a.invN);
                 },
-                [&](int, int, int j, float2 v) { if (valid) dst_row[j] = v; });
+                [&](int, int, int j, float2 v) { if (valid) store_stream(dst_row + j, v, a.stream_out); });
             __syncthreads();
         };
         if constexpr (row_regs_fast<L>()) {
@@ -248,7 +256,9 @@ __global__ void __launch_bounds__(RowCfg<L>::THREADS) k_rows(RowArgs a) {
         } else {
             for (int z = z0; z < z1; ++z)
                 plane(z, [&](auto&& src, auto&& dst) {
-                    FftRun<L, SIGN, typename Plan::radices, Plan::TPT>::run(tw_s, t, src, dst, lds);
+                    int tz = t;
+                    if constexpr (row_fresh<L>()) fresh(tz);
+                    FftRun<L, SIGN, typename Plan::radices, Plan::TPT>::run(tw_s, tz, src, dst, lds);
                 });
         }
     }
@@ -308,11 +318,11 @@ __global__ void __launch_bounds__((ColCfg<L, MODE>::THREADS)) k_cols(ColArgs a) 
         float2 ph = make_float2(1.0f, 0.0f);
         if constexpr (MODE == COL_ADJ) ph = a.phase[z];  // e^{+i phi_z} (sparse_phase_scale_kernel2)
         FftRun<L, SIGN, typename Plan::radices, Plan::TPT>::run(
-            tw_s, t, [&](int, int, int j) { return src[(size_t)j * W]; },
+            tw_s, t, [&](int, int, int j) { return load_stream(src + (size_t)j * W, MODE == COL_ADJ); },
             [&](int, int, int j, float2 v) {
                 if constexpr (MODE == COL_ADJ)
                     v = make_float2(v.x * ph.x - v.y * ph.y, v.y * ph.x + v.x * ph.y);
-                dst[(size_t)j * W] = v;
+                store_stream(dst + (size_t)j * W, v, MODE == COL_ADJ);
             },
             lds);
     } else if constexpr (MODE == COL_FWD) {
@@ -323,9 +333,9 @@ __global__ void __launch_bounds__((ColCfg<L, MODE>::THREADS)) k_cols(ColArgs a) 
         const int z = blockIdx.y;
         const int line = (blockIdx.x * kColStrip) >> a.lsh;
         const uint64_t* occ = a.occ ? a.occ + (size_t)z * L : nullptr;
-        // the strip's row bits in LDS (from the map, or all set without one)
+        // the strip's row bits in LDS
         __shared__ uint32_t rows_s[(L + 31) / 32];
-        for (int k = threadIdx.x; k < (L + 31) / 32; k += C::THREADS) rows_s[k] = occ ? 0u : ~0u;
+        for (int k = threadIdx.x; k < (L + 31) / 32; k += C::THREADS) rows_s[k] = 0u;
         __syncthreads();
         bool mine = false;
         if (occ) {
@@ -342,14 +352,23 @@ __global__ void __launch_bounds__((ColCfg<L, MODE>::THREADS)) k_cols(ColArgs a) 
         const float px = ph.x, py = -ph.y;
         const float2* src = a.in + (size_t)z * L * W + col;
         float2* dst = a.out + (size_t)z * L * W + col;
-        FftRun<L, SIGN, typename Plan::radices, Plan::TPT>::run(
-            tw_s, t,
-            [&](int, int, int j) {
-                if (!((rows_s[j >> 5] >> (j & 31)) & 1u)) return make_float2(0.0f, 0.0f);
-                float2 d = src[(size_t)j * W];
-                return make_float2(d.x * px - d.y * py, d.y * px + d.x * py);
-            },
-            [&](int, int, int j, float2 v) { dst[(size_t)j * W] = v; }, lds);
+        using Run = FftRun<L, SIGN, typename Plan::radices, Plan::TPT>;
+        auto load = [&](int j) {
+            const float2 d = src[(size_t)j * W];
+            return make_float2(d.x * px - d.y * py, d.y * px + d.x * py);
+        };
+        auto store = [&](int, int, int j, float2 v) { dst[(size_t)j * W] = v; };
+        // without a map there is no test (and no branch) per element: 99 against 151 us at 640^2 x 64,
+        // 77 against 87 at 512^2 x 100
+        if (!occ)
+            Run::run(tw_s, t, [&](int, int, int j) { return load(j); }, store, lds);
+        else
+            Run::run(
+                tw_s, t,
+                [&](int, int, int j) {
+                    return ((rows_s[j >> 5] >> (j & 31)) & 1u) ? load(j) : make_float2(0.0f, 0.0f);
+                },
+                store, lds);
     } else {  // COL_REAL: est = Re(IFFT(...)), r = est - meas, partial sum |r|^2
         const float2* src = a.in + col;
         double s = 0.0;
@@ -454,6 +473,7 @@ hipError_t fft_rows_adj(int L, const float2* rhat, const double* kappa, const fl
     RowArgs a{};
     a.out = out; a.nrows = H; a.twg = tw_inv; a.rhat = rhat; a.kappa = kappa; a.zlist = zlist;
     a.nz = nz; a.zchunk = zchunk; a.invN = invN;
+    a.stream_out = streams(L, H, nz);
     const int gy = (nz + zchunk - 1) / zchunk;
     switch (L) {
 #define X(n) case n: return launch_rows_t<n, 1, ROW_ADJ>(a, H, gy, s);

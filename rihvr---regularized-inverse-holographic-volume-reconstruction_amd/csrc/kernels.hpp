@@ -18,6 +18,13 @@ inline int line_shift(int W) {  // log2 L
     return lsh;
 }
 
+// Whether a volume is larger than the memory-side cache (256 MB), so that the next pass finds
+// nothing of it there and A^T's row pass writes it past the caches; its column pass always reads and
+// writes past them (nothing of a plane is used twice).  Row pass + column pass + prox of an
+// iteration: 1492 -> 1470 us at 1024^2 x 128, 413 -> 385 at 512^2 x 100, 453 -> 418 at 640^2 x 64, 309 ->
+// 297 at 1024^2 x 16, unchanged at 256^2 x 64; with the row pass past the caches at 512^2 x 100 393.
+inline bool streams(int W, int H, int nz) { return 8l * W * H * nz > (256l << 20); }
+
 // ---- FFT (fft_kernels.hip) -------------------------------------------------
 bool fft_length_supported(int L);
 // workgroups of a row pass over one chunk of planes of H rows of length L (0: no fixed plan)
