@@ -1195,7 +1195,11 @@ class ObjectCloud:
         got = ctypes.c_int64()
         _check(lib().rihvr_segmentation_objects(self._seg._h, arr, n, ctypes.byref(got)),
                "rihvr_segmentation_objects")
-        return [arr[i].as_dict() for i in range(n)]
+        # all fields at once through numpy (an object's conversion by ctypes takes 3 us)
+        cols = np.frombuffer(arr, np.dtype(Object), n)
+        c, w, hi, mean, size, label, box = (np.ascontiguousarray(cols[k]).tolist() for k, _ in Object._fields_)
+        return [dict(centroid=c[i], weighted_centroid=w[i], max_value=hi[i], mean_value=mean[i], num_voxels=size[i],
+                     label=label[i], bounds=box[i]) for i in range(n)]
 
     def blobSizeFilter(self, min_size) -> int:
         removed = ctypes.c_int64()
