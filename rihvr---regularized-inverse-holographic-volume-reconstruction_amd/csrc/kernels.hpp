@@ -98,6 +98,7 @@ enum ProxSlot {
     PS_TVX0 = 4,     // sum 2D TV of x0               (calcTVNorm2d of the momentum point)
     PS_NNZX0 = 5,    // count of x0 != 0
     PS_NNZY = 6,     // count of y != 0
+    PS_SKIPPED = 7,  // a wave's output rows that the scan for zero rows skipped
     PS_COUNT = 8
 };
 
@@ -114,6 +115,7 @@ struct ProxLaunch {
     double reg_tv;      // TV weight
     int n_tv;
     int row_chunk;      // output rows per wave of the mode-7 prox (<= 0: default)
+    bool scan = false;  // mode 7 with maps: look for runs of zero rows first (the same results)
     double* partial;    // [nwaves][PS_COUNT]
     // mode 7 only, all required ([nz][H] words, see the line occupancy above): the maps of
     // Y0 and YM (their clear lines are not read), of Y's current content (its zero lines

@@ -62,8 +62,10 @@ struct ProxDev {
     float2* Y;
     int W, H, nz;
     float s_mom, t, mu, sc, thr;
+    float m_lim, d_lim2;  // a row of g is quiet within these
     const float* s_mom_dev;  // when set, the momentum step is read from it (replays of captured graphs)
     int do_soft;
+    bool scan;
     int lsh;  // a map line is 2^lsh voxels of a row: 16 up to W = 1024, then 32, 64 (64 lines per row)
     ProxGeom geo;
     int nwaves;
@@ -134,6 +136,7 @@ template <int NTV> struct ProxWave {
     uint64_t plane_bits = 0;  // lines this wave set in the new map (its plane word's share)
     float acc_ls1 = 0.f, acc_ls2 = 0.f, acc_rs = 0.f, acc_l1 = 0.f, acc_tv = 0.f, acc_nnz = 0.f;
     unsigned nnzy = 0;  // output voxels != 0 (wave-uniform)
+    bool woke = false;  // a row since this was cleared had a lane above the threshold
     float smom = 0.f;  // the momentum step s of x0 = y0 + s (y0 - ym)
 
     static __device__ __forceinline__ int wrap_row(int tau, int H) {
@@ -283,6 +286,7 @@ template <int NTV> struct ProxWave {
         } else {
             yv = make_float2(yv.x + 0.0f, yv.y + 0.0f);
         }
+        woke |= live;
         if (o >= r0 && o < r1) {  // row o: the new map and the skipped writes
             uint64_t m = 0ull;
             if (live) {
@@ -382,7 +386,7 @@ template <int NTV> struct ProxWave {
 // its state needs more registers than 5 waves leave.
 template <int NTV> constexpr int prox_waves_per_simd() { return NTV <= 5 ? 5 : 1; }
 
-template <int NTV>
+template <int NTV, bool SCAN>
 __global__ void __launch_bounds__(64 * kProxWaves)
     __attribute__((amdgpu_waves_per_eu(prox_waves_per_simd<NTV>()))) k_prox_fl2d(ProxDev a) {
     using PW = ProxWave<NTV>;
@@ -423,41 +427,125 @@ __global__ void __launch_bounds__(64 * kProxWaves)
         if (__builtin_amdgcn_ballot_w64((xcol >> a.lsh) == l)) st.wlines |= 1ull << l;
         if (__builtin_amdgcn_ballot_w64(out_lane && (ocol >> a.lsh) == l)) st.outlines |= 1ull << l;
     }
-#pragma unroll
-    for (int p = 0; p < 2; ++p)
-#pragma unroll
-        for (int k = 0; k <= NTV; ++k) {
-            st.gd[p][k] = make_float4(0.f, 0.f, 0.f, 0.f);
-            st.yh[p][k] = make_float2(0.f, 0.f);
-        }
-    const int tau0 = r0 - (NTV > 0 ? NTV : 1);
     const int tau1 = r1 + NTV;  // inclusive
-    // the first two rows; every step then loads the row two ahead (U is even)
     st.y0p = (const char*)(a.Y0 + plane_off);
     st.ymp = (const char*)(a.YM + plane_off);
     st.gp = (const char*)(a.G + plane_off);
     st.yp = (char*)(a.Y + plane_off);
     st.rowb = (unsigned)W * (unsigned)sizeof(float2);
-    st.row_ld = PW::wrap_row(tau0, a.H);
-    st.row_wd = st.row_ld;
-    st.row_cur = st.row_ld;
     st.m0 = a.occ_y0 + zrow;
     st.mm = a.occ_ym + zrow;
     st.mold = a.occ_old + zrow;
-    st.row_old = PW::wrap_row(tau0 - NTV, a.H);
-    st.load_words(0, a.H);  // tau0
-    st.load_words(1, a.H);  // tau0 + 1
-    st.load_row(a, 0, xoff, true);  // tau0
-    st.load_row(a, 1, xoff, true);  // tau0 + 1
-    st.load_words(0, a.H);  // tau0 + 2
-    st.oold[0] = PW::uniform_word(st.mold, (unsigned)PW::wrap_row(tau0 - NTV - 1, a.H));
-    int tau = tau0;
-    for (; tau + U - 1 <= tau1; tau += U)
-        st.block(std::make_integer_sequence<int, U>{}, a, tau, r0, r1, xoff, ocol, out_lane,
-                 tau1, zrow, strip);
-    if (tau <= tau1)
-        st.tail(std::make_integer_sequence<int, U - 1>{}, tau1 - tau + 1, a, tau, r0, r1, xoff,
-                ocol, out_lane, tau1, zrow, strip);
+
+    // Runs of rows whose output is +0 for certain are found from g alone.  Where x0 = 0 and no dual
+    // is projected, a TV iteration replaces x-hat by an average of itself and its neighbours
+    // (y - mu sc div grad y = y + (sum of the 4 neighbours - 4 y) / 12), so |y| stays within the
+    // largest |x-hat| = t |g| of the 2 n_tv + 1 rows and columns around, and |grad y| within the largest
+    // |grad x-hat|; the duals, sums of up to n_tv gradients times sc, are then within
+    // n_tv sc t max|grad g|.  So with |g| <= lambda1 per component and |grad g| <= 12 lambda_TV / n_tv (the
+    // 4-vector of both components' x and y differences) over those rows and columns, no dual reaches 1,
+    // the output is below the threshold, and the row has no term in the sums.  A quiet row satisfies
+    // both, holds no x0 and no old output to clear; an output row with NTV quiet rows on each side is
+    // skipped.  The scan has a tenth of the TV levels' operations per row and is bound by
+    // reading g: at 1024^2 x 128 an iteration's prox takes 0.38 ms instead of 0.60 where 1e-4 of y is
+    // non-zero, 0.46 instead of 0.61 at 1e-3 to 3e-4.
+    constexpr int kAhead = 4;  // rows tested together, while the next ones load
+    // the first output row from od on that may be non-zero, r1 if none
+    auto scan = [&](int od) {
+        const int first = od - HX, last = r1 - 1 + NTV;  // rows that the output rows [od, r1) see
+        float2 cur[kAhead], nxt[kAhead], up = make_float2(0.f, 0.f);
+        int row = PW::wrap_row(first, a.H);
+        auto load = [&](float2 (&v)[kAhead]) {
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) {
+                v[k] = PW::at(st.gp, (unsigned)row * st.rowb, xoff);
+                row = PW::next_row(row, a.H);
+            }
+        };
+        load(cur);
+        uint64_t held = 0;  // bit i: row (64-row group) + i holds x0 or an old output
+        for (int rho = first; rho <= last; rho += kAhead) {
+            load(nxt);
+            const int i0 = (rho - first) & 63;
+            if (i0 == 0) {  // the maps' words of 64 rows, a lane each
+                const int r = wrapi(rho + lane, a.H);
+                const uint64_t w = ((st.m0[r] | st.mm[r]) & st.wlines) | (st.mold[r] & st.outlines);
+                held = __builtin_amdgcn_ballot_w64(w != 0);
+            }
+            bool loud[kAhead], any = false;
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) {
+                const float2 g = cur[k];
+                const float2 u = k > 0 ? cur[k > 0 ? k - 1 : 0] : rho > first ? up : g;
+                const float lx = g.x - lane_from_left(g.x), ly = g.y - lane_from_left(g.y);
+                const float ux = g.x - u.x, uy = g.y - u.y;
+                // (lane 0 has no left neighbour here; its dual reaches no output lane)
+                const float l2 = lane > 0 ? fmaf(lx, lx, ly * ly) : 0.0f;
+                const float d2 = fmaf(ux, ux, fmaf(uy, uy, l2));  // NaN where g is not finite
+                loud[k] = !(fmaxf(fabsf(g.x), fabsf(g.y)) <= a.m_lim) || !(d2 <= a.d_lim2);
+                any |= loud[k];
+            }
+            if (((held >> i0) & ((1u << kAhead) - 1u)) != 0 || __builtin_amdgcn_ballot_w64(any)) {
+#pragma unroll
+                for (int k = 0; k < kAhead; ++k)
+                    if (((held >> (i0 + k)) & 1u) || __builtin_amdgcn_ballot_w64(loud[k]))
+                        return min(max(od, rho + k - NTV), r1);
+            }
+            up = cur[kAhead - 1];
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) cur[k] = nxt[k];
+        }
+        return r1;
+    };
+
+    int oa = r0;    // output rows from here on are formed
+    int need = 16;  // quiet output rows before rows are scanned again
+    int skipped = 0;
+    for (;;) {
+        if constexpr (SCAN) {
+            const int od = oa;
+            oa = scan(od);
+            skipped += oa - od;
+            if (oa >= r1) break;
+            if (oa - od < 16) need *= 2;  // too little was skipped: less often from here
+        }
+        // the TV levels from output row oa on: the first two rows; every step then loads the row two
+        // ahead (U is even)
+        int tau = oa - (NTV > 0 ? NTV : 1);
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+            for (int k = 0; k <= NTV; ++k) {
+                st.gd[p][k] = make_float4(0.f, 0.f, 0.f, 0.f);
+                st.yh[p][k] = make_float2(0.f, 0.f);
+            }
+        st.y0rows = st.xrows = 0;
+        st.row_ld = PW::wrap_row(tau, a.H);
+        st.row_wd = st.row_ld;
+        st.row_cur = st.row_ld;
+        st.row_old = PW::wrap_row(tau - NTV, a.H);
+        st.load_words(0, a.H);  // tau
+        st.load_words(1, a.H);  // tau + 1
+        st.load_row(a, 0, xoff, true);  // tau
+        st.load_row(a, 1, xoff, true);  // tau + 1
+        st.load_words(0, a.H);  // tau + 2
+        st.oold[0] = PW::uniform_word(st.mold, (unsigned)PW::wrap_row(tau - NTV - 1, a.H));
+        int quiet = 0;  // output rows since one was above the threshold or had x0 near it
+        while (tau + U - 1 <= tau1 && (!SCAN || quiet < need)) {
+            st.woke = false;
+            st.block(std::make_integer_sequence<int, U>{}, a, tau, oa, r1, xoff, ocol, out_lane, tau1, zrow, strip);
+            tau += U;
+            if constexpr (SCAN) quiet = st.woke || (st.xrows & ((1u << (NTV + 4)) - 1u)) ? 0 : quiet + U;
+        }
+        if (SCAN && tau + U - 1 <= tau1) {
+            oa = max(oa, tau - NTV - 1);
+            continue;
+        }
+        if (tau <= tau1)
+            st.tail(std::make_integer_sequence<int, U - 1>{}, tau1 - tau + 1, a, tau, oa, r1, xoff, ocol, out_lane,
+                    tau1, zrow, strip);
+        break;
+    }
 
     if (st.plane_bits && lane == 0) atomicOr((unsigned long long*)&a.occ_new_planes[z], st.plane_bits);
     const double s_ls1 = wave_sum((double)st.acc_ls1);
@@ -475,7 +563,7 @@ __global__ void __launch_bounds__(64 * kProxWaves)
         p[PS_TVX0] = s_tv;
         p[PS_NNZX0] = s_nnz;
         p[PS_NNZY] = (double)st.nnzy;
-        p[7] = 0.0;
+        p[PS_SKIPPED] = (double)skipped;
     }
 }
 
@@ -714,6 +802,11 @@ static ProxDev make_dev(const ProxLaunch& a) {
     d.sc = a.reg_tv != 0.0 ? (float)(1 / (4 * 3 * a.t * a.reg_tv)) : 0.0f;
     d.thr = (float)(a.t * a.reg);
     d.do_soft = a.reg > 0.0;
+    // a part in a thousand covers the rounding of the TV levels and of t g
+    d.m_lim = (float)(0.999 * a.reg);
+    const double dl = a.n_tv > 0 && a.reg_tv != 0.0 ? 0.999 * 12.0 * std::fabs(a.reg_tv) / a.n_tv : 1e18;
+    d.d_lim2 = (float)(dl * dl);
+    d.scan = a.scan && a.reg > 0.0;  // without a threshold no output is 0 for certain
     d.lsh = line_shift(a.W);
     d.geo = prox_geom(a.W, a.H, a.n_tv, a.row_chunk);
     d.nwaves = d.geo.nstrips * d.geo.nchunks * a.nz;
@@ -728,13 +821,16 @@ static ProxDev make_dev(const ProxLaunch& a) {
 
 template <int NTV> static hipError_t launch_fl2d(const ProxDev& d, hipStream_t s) {
     dim3 grid((d.nwaves + kProxWaves - 1) / kProxWaves);
-    hipLaunchKernelGGL(k_prox_fl2d<NTV>, grid, dim3(64 * kProxWaves), 0, s, d);
+    if (d.scan)
+        hipLaunchKernelGGL((k_prox_fl2d<NTV, true>), grid, dim3(64 * kProxWaves), 0, s, d);
+    else
+        hipLaunchKernelGGL((k_prox_fl2d<NTV, false>), grid, dim3(64 * kProxWaves), 0, s, d);
     return hipGetLastError();
 }
 
 template <int NTV> static int fl2d_blocks_per_cu() {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_prox_fl2d<NTV>, 64 * kProxWaves, 0) != hipSuccess)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_prox_fl2d<NTV, false>, 64 * kProxWaves, 0) != hipSuccess)
         return 0;
     return nb;
 }

@@ -34,6 +34,18 @@ constexpr double kPi = 3.14159265358979323846;
 // 358, 385, 512 (512^2 x 100, 97 % -> 10 %); at 1 %, 598, 595 and 361.
 constexpr double kDenseFraction = 0.05;
 
+// The mode-7 prox's forms: rows with data skip work, the same after a scan for runs of zero rows, dense.
+enum class ProxForm { rows, scan, dense };
+// The scan's kernel forms a row 4 to 10 % slower than the one without it, and a wave that resumes after
+// a run forms 2 n_tv + 1 rows again, so it is taken below a non-zero fraction and from a number of rows
+// per wave where it gained: 1024^2 x 128, 1.8e-3 and falling, 205 rows, prox of 80 iterations 33.0
+// instead of 47.9 ms; 512^2 x 100, 2.8e-3, 103 rows, 0.254 instead of 0.237 ms each; 512^2 x 16, 9e-4,
+// 16 rows, 84 instead of 70 us.  How much is quiet depends on the data and the weights as well: a pass that
+// skipped less than kScanPays of the rows turns the scan off until y has half as many non-zeros.
+constexpr double kScanFraction = 2e-3;
+constexpr int kScanRows = 64;
+constexpr double kScanPays = 0.2;
+
 // scalar slots after reduction
 enum Slot { SL_PROX = 0, SL_RESID_A = 8, SL_RESID_M = 9, SL_FLAG = 10, SL_COUNT = 16 };
 
@@ -89,6 +101,7 @@ struct SolveState {
     int iters = 0;
     bool g_ready = false;     // G = A^T r of the current residual (else only R-hat is)
     double nnz_y = 0;         // non-zero voxels of y_{k-1} (mode 7; 0 before the first prox)
+    double scan_below = INFINITY;  // the nnz_y below which scanning for zero rows may pay again
 };
 
 }  // namespace
@@ -152,6 +165,7 @@ struct rihvr_ctx {
     bool groups_one_stream = false;  // run A^T, prox and A group by group on the main stream
     int prox_rows = 0;    // output rows per prox wave (0: default)
     int prox_rows_dense = 0;  // the same for the dense prox
+    long prox_strip_rows = 0;  // output rows of all of the sparse prox's strips
     // Captured iterations: the two halves of a queued-ahead iteration (prox + A, then the
     // hologram momentum + the next A^T) as HIP graphs, one per pointer and step combination
     // (the volume ring, the maps and the spectra rotate through at most 12), replayed with the
@@ -460,7 +474,7 @@ bool tv3d(const rihvr_ctx* c) { return c->ss.mode == RIHVR_MODE_FASTA_FUSED_LASS
 // the launches)
 rihvr_status apply_prox(rihvr_ctx* c, int mode, const float2* Y0, const float2* YM, float s_mom, const float2* G,
                         double t, float2* Y, const float* s_mom_dev = nullptr, bool enqueue = true,
-                        bool dense = false) {
+                        ProxForm form = ProxForm::rows) {
     ProxLaunch a;
     a.Y0 = Y0; a.YM = YM; a.G = G; a.Y = Y;
     a.W = c->W; a.H = c->H; a.nz = c->Nz;
@@ -470,6 +484,7 @@ rihvr_status apply_prox(rihvr_ctx* c, int mode, const float2* Y0, const float2* 
     a.reg_tv = (double)c->p.regularization_TV_param;
     a.n_tv = c->p.num_tv_iterations;
     a.row_chunk = c->prox_rows;
+    a.scan = form == ProxForm::scan;
     a.partial = c->partial;
     int rows;
     const int ky = ring_index(c, Y);
@@ -478,7 +493,7 @@ rihvr_status apply_prox(rihvr_ctx* c, int mode, const float2* Y0, const float2* 
         if (enqueue) RIHVR_TRY(timed(c, K_PROX, [&] { return prox_tv2_general(a, c->tvbuf, c->stream); }));
         rows = prox_tv2_num_blocks(c->W, c->H, c->Nz);
         if (ky >= 0) c->occ_valid[ky] = false;
-    } else if (mode == RIHVR_MODE_FASTA_FUSED_LASSO_2D && dense) {
+    } else if (mode == RIHVR_MODE_FASTA_FUSED_LASSO_2D && form == ProxForm::dense) {
         a.row_chunk = c->prox_rows_dense;
         if (enqueue) RIHVR_TRY(timed(c, K_PROX, [&] { return prox_fl2d_dense(a, c->stream); }));
         rows = prox_fl2d_num_waves(c->W, c->H, c->Nz, a.n_tv, c->prox_rows_dense);
@@ -523,7 +538,8 @@ rihvr_status apply_prox(rihvr_ctx* c, int mode, const float2* Y0, const float2* 
 // Same kernels, same arithmetic and the same partial-row layout as the one-stream
 // sequence A^T (all planes), prox (all planes), A (all planes).
 rihvr_status pipelined_pass(rihvr_ctx* c, const float2* Y0, const float2* YM, float s_mom, double t, float2* Yn,
-                            bool dense) {
+                            ProxForm form) {
+    const bool dense = form == ProxForm::dense;
     if (!c->groups_one_stream) {
         RIHVR_HIP(hipStreamWaitEvent(c->aux, c->ev_rhat, 0));
         for (int g = 0, g0 = 0; g < c->n_groups; ++g, g0 += c->pipe_planes) {
@@ -538,6 +554,7 @@ rihvr_status pipelined_pass(rihvr_ctx* c, const float2* Y0, const float2* YM, fl
     a.reg_tv = (double)c->p.regularization_TV_param;
     a.n_tv = c->p.num_tv_iterations;
     a.row_chunk = dense ? c->prox_rows_dense : c->prox_rows;
+    a.scan = form == ProxForm::scan;
     const int per_plane = prox_fl2d_num_waves(c->W, c->H, 1, a.n_tv, a.row_chunk);
     const uint64_t* o0 = occ_of(c, Y0);
     const uint64_t* om = occ_of(c, YM);
@@ -728,6 +745,7 @@ rihvr_status create_impl(const rihvr_params* params, const rihvr_schedule* sch, 
     RIHVR_TRY(dalloc(&c->twiH, c->H));
     c->dense_ok = params->mode == RIHVR_MODE_FASTA_FUSED_LASSO_2D && !tv_general;
     c->prox_rows_dense = c->prox_rows;
+    c->prox_strip_rows = (long)prox_fl2d_num_waves(c->W, c->H, c->Nz, std::min(params->num_tv_iterations, 10), c->H) * c->H;
     // rows that a schedule gives hold for both forms, except where they are the rule's own (a
     // schedule read back from a context)
     if (c->dense_ok && (prow < 0 || prow == prox_fl2d_auto_rows(c->W, c->H, c->Nz, params->num_tv_iterations)))
@@ -980,33 +998,38 @@ rihvr_status iterate_impl(rihvr_ctx* c, int n_it, rihvr_stats* st, bool last_f_b
         float2* YM = c->Yb[c->iym];
         bool queued = false;  // the accepted-iteration work is queued
         const double a1 = (1.0 + std::sqrt(1.0 + 4.0 * alpha0 * alpha0)) / 2.0;  // alpha_{k+1} without a restart
-        const bool dense = c->dense_ok && s.nnz_y >= kDenseFraction * (double)c->V;
+        ProxForm form = ProxForm::rows;
+        if (c->dense_ok && s.nnz_y >= kDenseFraction * (double)c->V)
+            form = ProxForm::dense;
+        else if (c->dense_ok && s.nnz_y > 0 && s.nnz_y < std::min(s.scan_below, kScanFraction * (double)c->V) &&
+                 c->prox_rows >= kScanRows)
+            form = ProxForm::scan;
         for (;;) {
             const bool use_graph = ahead && c->graphs && !c->tm.on;
             if (!s.g_ready && mode == RIHVR_MODE_FASTA_FUSED_LASSO_2D && c->n_groups > 1) {
-                RIHVR_TRY(pipelined_pass(c, Y0, YM, s.s_mom, s.t, Yn, dense));
+                RIHVR_TRY(pipelined_pass(c, Y0, YM, s.s_mom, s.t, Yn, form));
             } else {
                 if (!s.g_ready)
                     for (int g0 = 0; g0 < c->Nz; g0 += c->pipe_planes)
                         RIHVR_TRY(adjoint_group(c, c->G, g0, std::min(c->pipe_planes, c->Nz - g0), c->stream));
                 if (use_graph) {
                     // the steps that the replayed graphs read, and the map that the prox builds
-                    const bool maps = mode == RIHVR_MODE_FASTA_FUSED_LASSO_2D && !c->tvbuf && !dense;
+                    const bool maps = mode == RIHVR_MODE_FASTA_FUSED_LASSO_2D && !c->tvbuf && form != ProxForm::dense;
                     RIHVR_HIP(begin_iteration(c->d_smom, s.s_mom, c->d_step, (alpha0 - 1) / a1, c->occ_tmp,
                                               maps ? (long)map_words(c) : 0L, c->stream));
                     const std::vector<const void*> key = {
                         Y0, YM, Yn, c->G, c->hX, c->occ[0], c->occ[1], c->occ[2], c->occ_tmp,
                         (const void*)(intptr_t)(c->occ_valid[0] | (c->occ_valid[1] << 1) | (c->occ_valid[2] << 2)),
-                        (const void*)(intptr_t)(mode | (dense ? 256 : 0)), (const void*)(uintptr_t)weight_bits(c)};
+                        (const void*)(intptr_t)(mode | ((int)form << 8)), (const void*)(uintptr_t)weight_bits(c)};
                     RIHVR_TRY(graph_run(
                         c, 0, key, s.t,
                         [&] {
-                            RIHVR_TRY(apply_prox(c, mode, Y0, YM, s.s_mom, c->G, s.t, Yn, c->d_smom, true, dense));
+                            RIHVR_TRY(apply_prox(c, mode, Y0, YM, s.s_mom, c->G, s.t, Yn, c->d_smom, true, form));
                             return apply_forward(c, Yn, c->hX);
                         },
-                        [&] { return apply_prox(c, mode, Y0, YM, s.s_mom, c->G, s.t, Yn, c->d_smom, false, dense); }));
+                        [&] { return apply_prox(c, mode, Y0, YM, s.s_mom, c->G, s.t, Yn, c->d_smom, false, form); }));
                 } else {
-                    RIHVR_TRY(apply_prox(c, mode, Y0, YM, s.s_mom, c->G, s.t, Yn, nullptr, true, dense));
+                    RIHVR_TRY(apply_prox(c, mode, Y0, YM, s.s_mom, c->G, s.t, Yn, nullptr, true, form));
                     RIHVR_TRY(apply_forward(c, Yn, c->hX));
                 }
             }
@@ -1106,6 +1129,8 @@ rihvr_status iterate_impl(rihvr_ctx* c, int n_it, rihvr_stats* st, bool last_f_b
         }
         if (i == n_it) break;  // stopped at the objective target
         s.nnz_y = c->h_scal[SL_PROX + PS_NNZY];
+        if (form == ProxForm::scan && c->h_scal[SL_PROX + PS_SKIPPED] < kScanPays * (double)c->prox_strip_rows)
+            s.scan_below = s.nnz_y / 2;
         const double rs = c->h_scal[SL_PROX + PS_RESTART];
         const bool restart = rs > 0;  // :4481
         if (restart) alpha0 = 1;
