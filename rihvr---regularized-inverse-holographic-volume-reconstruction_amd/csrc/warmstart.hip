@@ -54,6 +54,19 @@ __device__ __forceinline__ unsigned short f2bf(float f) {
     return (unsigned short)(u >> 16);
 }
 
+// The products of two taps in one MFMA (K = 32): lane group q holds channels 8 (q & 1) .. + 7 of the
+// first tap (q < 2) or the second in 16 bytes, of voxel r16 in a and of output channel r16 in b.
+// Half the matrix instructions and LDS reads of one tap at K = 16, and 16 lanes read 256 contiguous
+// bytes instead of every other 8.  A single tap left over runs with zeros in the second's place: a
+// K = 16 MFMA right after a K = 32 one on the same accumulator gave results that differed from run to
+// run.  One tap at a time, then two: prediction at 128 x 1024^2 19.8 -> 18.0 ms (the 16-channel layers
+// 8.0 -> 7.8 and 3.63 -> 3.46, now held by the staging, the others 5.3 -> 3.9), loss and gradient at
+// 64 x 128^2 1.96 -> 1.71 ms.
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ f4 mfma_taps(const uint4& a, const uint4& b, const f4& c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, a), __builtin_bit_cast(bf8, b), c, 0, 0, 0);
+}
+
 struct ConvGeo {
     int D, H, W;  // full-resolution grid of the output and of in0
     int C0, C1;   // channels of in0 (full resolution) and of in1 (half resolution, read upsampled)
@@ -97,9 +110,9 @@ __global__ void __launch_bounds__(kFwdThreads) k_conv_fwd(const unsigned short* 
     constexpr int TY = 4 * ROWS, HY = TY + 2, HALO = HY * kHX;
     constexpr int MT = 4 * ROWS;                       // M-tiles per wave
     constexpr int NTMAX = ROWS == 1 ? 4 : 1;           // N-tiles per wave at most
-    __shared__ uint4 halo[HALO * 2];     // [row][x][16 ch] as two 16-byte halves per voxel
+    __shared__ uint4 halo[HALO * 2];     // [half of 8 ch][row][x]
     constexpr int CBM = ROWS == 2 ? 16 : kMaxCB;  // ROWS = 2 runs CB = 16 only (conv_forward)
-    __shared__ s4 wl[9 * CBM * 4];       // [tap of the slab][co][4 groups of 4 ci]
+    __shared__ uint4 wl[9 * CBM * 2];    // [half of 8 ci][tap of the slab][co]
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int q = lane >> 4, r16 = lane & 15;
     const int nxt = (g.W + 63) >> 6;
@@ -115,15 +128,15 @@ __global__ void __launch_bounds__(kFwdThreads) k_conv_fwd(const unsigned short* 
 #pragma unroll
         for (int n = 0; n < NTMAX; ++n) acc[m][n] = f4{0.f, 0.f, 0.f, 0.f};
     const int nchunks = Cin >> 4;
-    const unsigned short* hs = (const unsigned short*)halo;
     // The halo and weight slots this thread stages are the same in every stage: their source
     // offsets (halo: within a plane and chunk of in0, or of in1 at half resolution, -1 outside
     // the grid, -2 no slot; weights: within a dz slab and chunk, -1 no slot) are computed once,
-    // and a stage adds its base.  The weight slab is stored [tap][co][4 groups of 4 ci] with co
-    // stride CB, so slot e of the slab is wl[e].  (Offsets are 32-bit: conv_forward checks that
+    // and a stage adds its base.  Halo and weights lie as two arrays of 16-byte channel halves, so
+    // that 16 lanes reading one half of 16 voxels (or output channels) read 256 contiguous bytes.
+    // (Offsets are 32-bit: conv_forward checks that
     // they fit.)
     constexpr int kPer = (HALO * 2 + kFwdThreads - 1) / kFwdThreads;
-    constexpr int kPerW = (9 * CBM * 4 + kFwdThreads - 1) / kFwdThreads;
+    constexpr int kPerW = (9 * CBM * 2 + kFwdThreads - 1) / kFwdThreads;
     int hoff0[kPer], hoff1[kPer], woff[kPerW];
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
@@ -142,9 +155,9 @@ __global__ void __launch_bounds__(kFwdThreads) k_conv_fwd(const unsigned short* 
     for (int k = 0; k < kPerW; ++k) {
         const int e = threadIdx.x + k * kFwdThreads;
         woff[k] = -1;
-        if (e < 9 * g.CB * 4) {
-            const int qq = e & 3, co = (e >> 2) % g.CB, tt = (e >> 2) / g.CB;
-            woff[k] = (tt * g.Cout + co0 + co) * Cin + qq * 4;
+        if (e < 9 * g.CB * 2) {
+            const int co = (e >> 1) % g.CB, tt = (e >> 1) / g.CB;
+            woff[k] = (tt * g.Cout + co0 + co) * Cin + (e & 1) * 8;
         }
     }
     for (int c = 0; c < nchunks; ++c) {
@@ -165,29 +178,52 @@ __global__ void __launch_bounds__(kFwdThreads) k_conv_fwd(const unsigned short* 
 #pragma unroll
             for (int k = 0; k < kPer; ++k) {
                 const int e = threadIdx.x + k * kFwdThreads;
-                if (e < HALO * 2) halo[e] = v[k];
+                if (e < HALO * 2) halo[(e & 1) * HALO + (e >> 1)] = v[k];
             }
             const unsigned short* wbase = w + (size_t)((dz + 1) * 9) * g.Cout * Cin + c * 16;
 #pragma unroll
             for (int k = 0; k < kPerW; ++k)
-                if (woff[k] >= 0) wl[threadIdx.x + k * kFwdThreads] = *(const s4*)(wbase + woff[k]);
+                if (woff[k] >= 0) {
+                    const int e = threadIdx.x + k * kFwdThreads;
+                    s4* slot = (s4*)&wl[(e & 1) * 9 * g.CB + (e >> 1)];
+                    slot[0] = *(const s4*)(wbase + woff[k]);  // (a caller's weights may be 8-byte aligned)
+                    slot[1] = *(const s4*)(wbase + woff[k] + 4);
+                }
             __syncthreads();
+            // taps (0, 1) .. (6, 7), two to an MFMA
 #pragma unroll
-            for (int tt = 0; tt < 9; ++tt) {
-                const int dy = tt / 3 - 1, dx = tt % 3 - 1;
-                s4 a[MT];
+            for (int tt = 0; tt < 8; tt += 2) {
+                constexpr auto tap = [](int t) { return (t / 3) * kHX + t % 3; };
+                const int lane0 = (q & 1) * HALO + r16 + (q >> 1) * (tap(tt + 1) - tap(tt));
+                uint4 a[MT];
+#pragma unroll
+                for (int m = 0; m < MT; ++m)
+                    a[m] = halo[lane0 + (wave * ROWS + (m >> 2)) * kHX + (m & 3) * 16 + tap(tt)];
+#pragma unroll
+                for (int n = 0; n < NTMAX; ++n) {
+                    if (n < NT) {
+                        const uint4 b = wl[((q & 1) * 9 + tt + (q >> 1)) * g.CB + n * 16 + r16];
+#pragma unroll
+                        for (int m = 0; m < MT; ++m) acc[m][n] = mfma_taps(a[m], b, acc[m][n]);
+                    }
+                }
+            }
+            {  // tap 8 alone: zeros in the second tap's place
+                const uint4 zero = make_uint4(0, 0, 0, 0);
+                const int lane0 = (q & 1) * HALO + r16;
+                uint4 a[MT];
 #pragma unroll
                 for (int m = 0; m < MT; ++m) {
-                    const int row = (wave * ROWS + (m >> 2) + dy + 1) * kHX;
-                    a[m] = *(const s4*)(hs + (size_t)(row + (m & 3) * 16 + r16 + dx + 1) * 16 + q * 4);
+                    a[m] = halo[lane0 + (wave * ROWS + (m >> 2) + 2) * kHX + (m & 3) * 16 + 2];
+                    if (q >= 2) a[m] = zero;
                 }
 #pragma unroll
                 for (int n = 0; n < NTMAX; ++n) {
                     if (n < NT) {
-                        const s4 b = wl[(tt * g.CB + n * 16 + r16) * 4 + q];
+                        uint4 b = wl[((q & 1) * 9 + 8) * g.CB + n * 16 + r16];
+                        if (q >= 2) b = zero;
 #pragma unroll
-                        for (int m = 0; m < MT; ++m)
-                            acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[m], b, acc[m][n], 0, 0, 0);
+                        for (int m = 0; m < MT; ++m) acc[m][n] = mfma_taps(a[m], b, acc[m][n]);
                     }
                 }
             }
@@ -317,8 +353,7 @@ k_conv_dma(const unsigned short* __restrict__ in0,
             hoff0[i] = -2;
             if (e < HALO * 2) {
                 // slot e: channel half e / HALO of voxel e % HALO (the halves in two arrays, so
-                // that 16 lanes reading one 8-byte chunk of 16 voxels meet 2-way bank conflicts,
-                // not the 4-way of 32-byte voxel records)
+                // that 16 lanes reading one half of 16 voxels read contiguous bytes)
                 const int vox = e % HALO, half = e / HALO;
                 const int ry = vox / kHX, col = vox - ry * kHX;
                 // the columns x-parity-split (even ones, then odd ones)
@@ -412,19 +447,17 @@ k_conv_dma(const unsigned short* __restrict__ in0,
     auto compute = [&](int st, const uint4* hb, const uint4* wb) {
         const int c = st / 3, d = st - 3 * (st / 3);
         const bool hi = c * 16 >= g.C0;
-        const unsigned short* hs = (const unsigned short*)hb;
-        const s4* wq = (const s4*)wb;
         if (PAR && hi) {
+            // taps (oy, ox = 0) and (oy, ox = 1) to an MFMA
 #pragma unroll
-            for (int oo = 0; oo < 4; ++oo) {
-                const int oy = oo >> 1, ox = oo & 1;
-                s4 a[MT];
+            for (int oy = 0; oy < 2; ++oy) {
+                uint4 a[MT];
 #pragma unroll
                 for (int m = 0; m < MT; ++m) {
                     const int yr = wave * ROWS + (m >> 2);
                     const int hrow = (yr >> 1) + (yr & 1) + oy;
-                    const int hcol = 16 * ((m & 3) >> 1) + r16 + (m & 1) + ox;
-                    a[m] = *(const s4*)(hs + ((size_t)(q >> 1) * HALO2 + hrow * kHX2 + hcol) * 8 + (q & 1) * 4);
+                    const int hcol = 16 * ((m & 3) >> 1) + r16 + (m & 1) + (q >> 1);
+                    a[m] = hb[(q & 1) * HALO2 + hrow * kHX2 + hcol];
                 }
 #pragma unroll
                 for (int n = 0; n < NTMAX; ++n) {
@@ -432,9 +465,9 @@ k_conv_dma(const unsigned short* __restrict__ in0,
 #pragma unroll
                         for (int m = 0; m < MT; ++m) {
                             const int yr = wave * ROWS + (m >> 2);
-                            const int sl = ((yr & 1) * 2 + (m & 1)) * 4 + oo;
-                            const s4 bb = wq[((q >> 1) * 16 * g.CB + sl * g.CB + n * 16 + r16) * 2 + (q & 1)];
-                            acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[m], bb, acc[m][n], 0, 0, 0);
+                            const int sl = ((yr & 1) * 2 + (m & 1)) * 4 + oy * 2 + (q >> 1);
+                            const uint4 bb = wb[((q & 1) * 16 + sl) * g.CB + n * 16 + r16];
+                            acc[m][n] = mfma_taps(a[m], bb, acc[m][n]);
                         }
                     }
                 }
@@ -442,26 +475,50 @@ k_conv_dma(const unsigned short* __restrict__ in0,
             return;
         }
         (void)d;
+        // voxel of the halo that M-tile m's lane r16 reads at tap t, without r16 (PAR: the columns of
+        // one x parity are contiguous)
+        auto at = [&](int m, int t) {
+            const int row = (wave * ROWS + (m >> 2) + t / 3) * kHX;
+            if (!PAR) return row + (m & 3) * 16 + t % 3;
+            const int sx = (m & 1) + t % 3;
+            return row + 16 * ((m & 3) >> 1) + (sx & 1) * (kHX / 2) + (sx >> 1);
+        };
+        // taps (0, 1) .. (6, 7), two to an MFMA
 #pragma unroll
-        for (int tt = 0; tt < 9; ++tt) {
-            const int dy = tt / 3 - 1, dx = tt % 3 - 1;
-            s4 a[MT];
+        for (int tt = 0; tt < 8; tt += 2) {
+            uint4 a[MT];
 #pragma unroll
             for (int m = 0; m < MT; ++m) {
-                const int row = (wave * ROWS + (m >> 2) + dy + 1) * kHX;
-                const int hc = xcol(m, r16) + dx + 1;
-                const int col = PAR ? (hc & 1) * (kHX / 2) + (hc >> 1) : hc;
-                a[m] = PAR ? *(const s4*)(hs + ((size_t)(q >> 1) * HALO + row + col) * 8 + (q & 1) * 4)
-                           : *(const s4*)(hs + (size_t)(row + col) * 16 + q * 4);
+                const int vox = at(m, tt) + (q >> 1) * (at(m, tt + 1) - at(m, tt)) + r16;
+                a[m] = PAR ? hb[(q & 1) * HALO + vox] : hb[vox * 2 + (q & 1)];
             }
 #pragma unroll
             for (int n = 0; n < NTMAX; ++n) {
                 if (n < NT) {
-                    const s4 bb = PAR ? wq[((q >> 1) * 9 * g.CB + tt * g.CB + n * 16 + r16) * 2 + (q & 1)]
-                                      : wq[(tt * g.CB + n * 16 + r16) * 4 + q];
+                    const int wv = (tt + (q >> 1)) * g.CB + n * 16 + r16;
+                    const uint4 bb = PAR ? wb[(q & 1) * 9 * g.CB + wv] : wb[wv * 2 + (q & 1)];
 #pragma unroll
-                    for (int m = 0; m < MT; ++m)
-                        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[m], bb, acc[m][n], 0, 0, 0);
+                    for (int m = 0; m < MT; ++m) acc[m][n] = mfma_taps(a[m], bb, acc[m][n]);
+                }
+            }
+        }
+        {  // tap 8 alone: zeros in the second tap's place
+            const uint4 zero = make_uint4(0, 0, 0, 0);
+            uint4 a[MT];
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                const int vox = at(m, 8) + r16;
+                a[m] = PAR ? hb[(q & 1) * HALO + vox] : hb[vox * 2 + (q & 1)];
+                if (q >= 2) a[m] = zero;
+            }
+#pragma unroll
+            for (int n = 0; n < NTMAX; ++n) {
+                if (n < NT) {
+                    const int wv = 8 * g.CB + n * 16 + r16;
+                    uint4 bb = PAR ? wb[(q & 1) * 9 * g.CB + wv] : wb[wv * 2 + (q & 1)];
+                    if (q >= 2) bb = zero;
+#pragma unroll
+                    for (int m = 0; m < MT; ++m) acc[m][n] = mfma_taps(a[m], bb, acc[m][n]);
                 }
             }
         }
