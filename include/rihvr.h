@@ -266,6 +266,19 @@ rihvr_status rihvr_set_timing(rihvr_ctx* ctx, int32_t enable);
 rihvr_status rihvr_get_timing(rihvr_ctx* ctx, rihvr_kernel_time* out, int32_t capacity,
                               int32_t* count);
 
+/* What a context's solves did since it was created, for diagnosis (two solves that disagree: the
+ * per-iteration decisions are in rihvr_stats). */
+typedef struct rihvr_counters {
+    int64_t late_scalars;  /* iterations whose scalars were not yet the host's when they were due: taken
+                              by a copy instead (expected to stay 0) */
+    int64_t prox_rows;     /* iterations of the fused mode-7 prox in its sparse form, */
+    int64_t prox_scan;     /* ... the same after a scan for runs of zero rows, */
+    int64_t prox_dense;    /* ... and in its dense form */
+    int64_t scan_skipped;  /* rows (of the waves' strips) that the scans skipped */
+    int64_t graphs;        /* captured graphs held now */
+} rihvr_counters;
+rihvr_status rihvr_get_counters(const rihvr_ctx* ctx, rihvr_counters* out);
+
 /* The parameter set the context was created with. */
 rihvr_status rihvr_get_params(const rihvr_ctx* ctx, rihvr_params* out);
 

@@ -37,7 +37,7 @@ STATUS_NAMES = {
 EXPORTED = ("rihvr_abi_version", "rihvr_status_string", "rihvr_create", "rihvr_destroy",
             "rihvr_reconstruct", "rihvr_begin", "rihvr_iterate", "rihvr_finish", "rihvr_set_timing",
             "rihvr_get_timing", "rihvr_get_volume", "rihvr_get_plane", "rihvr_set_stepsize",
-            "rihvr_get_estimate", "rihvr_forward", "rihvr_adjoint", "rihvr_prox", "rihvr_get_params",
+            "rihvr_get_estimate", "rihvr_forward", "rihvr_adjoint", "rihvr_prox", "rihvr_get_params", "rihvr_get_counters",
             "rihvr_snapshot", "rihvr_read_param_file", "rihvr_read_image", "rihvr_prepare_hologram",
             "rihvr_write_tiff8", "rihvr_write_hologram", "rihvr_save_sparse", "rihvr_save_projections",
             "rihvr_save_planes", "rihvr_reconstruct_batch", "rihvr_write_png8", "rihvr_background_mean",
@@ -144,6 +144,16 @@ class Schedule(ctypes.Structure):
     @classmethod
     def make(cls, fft_path=0, max_radix=16, zchunk_fwd=0, zchunk_adj=0, prox_rows=0, graphs=1):
         return cls(int(fft_path), int(max_radix), int(zchunk_fwd), int(zchunk_adj), int(prox_rows), int(graphs), 0.0)
+
+    def as_dict(self) -> dict:
+        return {k: getattr(self, k) for k, _ in self._fields_}
+
+
+class Counters(ctypes.Structure):
+    """Mirror of ``rihvr_counters`` (include/rihvr.h): what a context's solves did."""
+
+    _fields_ = [(k, ctypes.c_int64) for k in ("late_scalars", "prox_rows", "prox_scan", "prox_dense", "scan_skipped",
+                                              "graphs")]
 
     def as_dict(self) -> dict:
         return {k: getattr(self, k) for k, _ in self._fields_}
@@ -331,6 +341,8 @@ def lib():
         L.rihvr_prox.restype = st
         L.rihvr_get_params.argtypes = [vp, _P(Params)]
         L.rihvr_get_params.restype = st
+        L.rihvr_get_counters.argtypes = [vp, _P(Counters)]
+        L.rihvr_get_counters.restype = st
         L.rihvr_snapshot.argtypes = [vp]
         L.rihvr_snapshot.restype = st
         cp, i32p = ctypes.c_char_p, _P(ctypes.c_int32)
@@ -696,6 +708,12 @@ class SparseCompressiveHolo:
         s = Schedule()
         _check(lib().rihvr_get_schedule(self._ctx, ctypes.byref(s)), "rihvr_get_schedule")
         return s.as_dict()
+
+    def counters(self) -> dict:
+        """rihvr_get_counters: late scalars, iterations by prox form, rows skipped, graphs held."""
+        n = Counters()
+        _check(lib().rihvr_get_counters(self._ctx, ctypes.byref(n)), "rihvr_get_counters")
+        return n.as_dict()
 
     # -- lifecycle --------------------------------------------------------
     def destroy(self):

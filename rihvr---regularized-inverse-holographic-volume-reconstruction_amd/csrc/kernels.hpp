@@ -202,12 +202,21 @@ hipError_t holo_spec(const float2* parts, int nparts, long stride, int W, int H,
 // out = f * in
 hipError_t holo_scale(const float2* in, float2* out, long n, float f, hipStream_t s);
 
+// A block of n scalars that a reduction hands to the host: src's last value is raised by 1 (the number
+// of blocks handed over), the block is copied to snap (device) and host (pinned), the last value of host
+// after the others have reached it.
+struct Publish {
+    double* src;
+    double* snap;
+    double* host;
+    int n;
+};
+
 // sums rows of partial [nrows][ncols] into out[ncols] (fixed order: deterministic);
-// work holds kReduceBlocks * ncols doubles.  Then pub_dst[0 .. pub_n) = pub_src[0 .. pub_n), when
-// set (pinned host memory; it may include out).
+// work holds kReduceBlocks * ncols doubles.  Then publishes a block, when given (it may include out).
 constexpr int kReduceBlocks = 64;
 hipError_t reduce_partials(const double* partial, int nrows, int ncols, double* work, double* out, hipStream_t s,
-                           const double* pub_src = nullptr, double* pub_dst = nullptr, int pub_n = 0);
+                           const Publish* pub = nullptr);
 
 // flags[0] = 1 if any element of a [n] complex array is not finite
 hipError_t check_finite(const float2* a, long n, int* flag, hipStream_t s);

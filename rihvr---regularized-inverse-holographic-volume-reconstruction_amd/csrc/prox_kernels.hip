@@ -1722,12 +1722,13 @@ __global__ void __launch_bounds__(kReduceThreads) k_reduce_rows(const double* __
     }
 }
 
-// The sums of all columns by one workgroup, in a fixed order; then pub_dst[0 .. pub_n) = pub_src
-// (host memory that the device writes: the scalars reach the host with the sums, without a copy).
+// The sums of all columns by one workgroup, in a fixed order; then the block of scalars for the host
+// (memory that the device writes: the scalars reach the host with the sums, without a copy).  The
+// block's number goes last, once the other values are visible to the host: a reader that finds the
+// number it expects has that block whole, and any other is seen to be late.
 constexpr int kReduceOneThreads = 1024;
 __global__ void __launch_bounds__(kReduceOneThreads)
-k_reduce_one(const double* __restrict__ partial, int nrows, int ncols, double* out, const double* pub_src,
-             double* pub_dst, int pub_n) {
+k_reduce_one(const double* __restrict__ partial, int nrows, int ncols, double* out, Publish pub) {
     __shared__ double red[PS_COUNT][kReduceOneThreads / 64];
     double acc[PS_COUNT];
 #pragma unroll
@@ -1750,10 +1751,20 @@ k_reduce_one(const double* __restrict__ partial, int nrows, int ncols, double* o
         for (int w = 0; w < kReduceOneThreads / 64; ++w) r += red[threadIdx.x][w];
         out[threadIdx.x] = r;
     }
-    if (!pub_dst) return;
+    if (!pub.host) return;
     __threadfence();
     __syncthreads();
-    if ((int)threadIdx.x < pub_n) pub_dst[threadIdx.x] = pub_src[threadIdx.x];
+    const int i = threadIdx.x, last = pub.n - 1;
+    double v = 0.0;
+    if (i <= last) {
+        v = pub.src[i];
+        if (i == last) pub.src[i] = v += 1.0;
+        pub.snap[i] = v;
+        if (i < last) pub.host[i] = v;
+    }
+    __threadfence_system();
+    __syncthreads();
+    if (i == last) __hip_atomic_store(&pub.host[i], v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // One workgroup takes up to this many rows by itself: a launch less, which is what a reduction
@@ -1762,8 +1773,9 @@ k_reduce_one(const double* __restrict__ partial, int nrows, int ncols, double* o
 constexpr int kReduceOneRows = 4096;
 
 hipError_t reduce_partials(const double* partial, int nrows, int ncols, double* work, double* out, hipStream_t s,
-                           const double* pub_src, double* pub_dst, int pub_n) {
-    if (ncols < 1 || ncols > PS_COUNT || nrows < 0 || pub_n > kReduceOneThreads) return hipErrorInvalidValue;
+                           const Publish* pub) {
+    if (ncols < 1 || ncols > PS_COUNT || nrows < 0 || (pub && (pub->n < 1 || pub->n > kReduceOneThreads)))
+        return hipErrorInvalidValue;
     if (nrows > kReduceOneRows) {
         const int rpb = (nrows + kReduceBlocks - 1) / kReduceBlocks;
         const int nb = (nrows + rpb - 1) / rpb;
@@ -1773,8 +1785,8 @@ hipError_t reduce_partials(const double* partial, int nrows, int ncols, double* 
         partial = work;
         nrows = nb;
     }
-    hipLaunchKernelGGL(k_reduce_one, dim3(1), dim3(kReduceOneThreads), 0, s, partial, nrows, ncols, out, pub_src,
-                       pub_dst, pub_n);
+    hipLaunchKernelGGL(k_reduce_one, dim3(1), dim3(kReduceOneThreads), 0, s, partial, nrows, ncols, out,
+                       pub ? *pub : Publish{});
     return hipGetLastError();
 }
 

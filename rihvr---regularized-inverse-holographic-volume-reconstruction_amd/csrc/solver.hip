@@ -46,8 +46,8 @@ constexpr double kScanFraction = 2e-3;
 constexpr int kScanRows = 64;
 constexpr double kScanPays = 0.2;
 
-// scalar slots after reduction
-enum Slot { SL_PROX = 0, SL_RESID_A = 8, SL_RESID_M = 9, SL_FLAG = 10, SL_COUNT = 16 };
+// scalar slots after reduction; SL_SEQ, the last: the number of blocks handed to the host
+enum Slot { SL_PROX = 0, SL_RESID_A = 8, SL_RESID_M = 9, SL_FLAG = 10, SL_SEQ = 15, SL_COUNT = 16 };
 
 #define RIHVR_HIP(call)                                                   \
     do {                                                                  \
@@ -115,7 +115,7 @@ struct rihvr_ctx {
     hipStream_t aux = nullptr;     // A^T of the next plane group while prox and A run on `stream`
     std::vector<hipEvent_t> ev_adj;  // per plane group: its G planes are written (on aux)
     hipEvent_t ev_rhat = nullptr;    // R-hat is written (on stream)
-    hipEvent_t ev_scal = nullptr;    // the scalars of the last prox + A are in h_scal
+    hipEvent_t ev_scal = nullptr;    // the scalars of the last prox + A are published
     // volumes
     float2* Yb[3] = {nullptr, nullptr, nullptr};  // ring of prox outputs
     int iy = 0, iy0 = 1, iym = 2;                 // y_k, y_{k-1}, y_{k-2}
@@ -157,7 +157,12 @@ struct rihvr_ctx {
     long partial_rows = 0, holo_rows = 0;
     double* scal = nullptr;
     double* red_work = nullptr;  // first-pass sums of reduce_partials
+    double* scal_pub = nullptr;  // the block of scalars that A's last reduction published
+    // pinned: the published block as the device writes it, then the target of stream-ordered copies
     double* h_scal = nullptr;
+    double sc[16] = {};          // the scalars the host works with
+    double published = 0;        // blocks published by the work queued so far
+    rihvr_counters counters{};   // what the solves so far did
     int* dflag = nullptr;
     int zchunk_adj = 8, zchunk_fwd = 8, nparts = 1;
     int pipe_planes = 1;  // planes per pipeline group (a multiple of the z chunks)
@@ -187,6 +192,9 @@ struct rihvr_ctx {
     // first attempt of those iterations is rejected as if its ratio were above 1, so the
     // backtracking paths can be exercised; never set in normal use
     uint64_t test_backtracks = 0;
+    // the same for RIHVR_TEST_LATE_SCALARS: in those iterations the host finds the block published before
+    uint64_t test_late = 0;
+    double test_prev[16] = {};
     Timer tm;
     SolveState ss;
 };
@@ -304,25 +312,51 @@ rihvr_status resolve_timing(rihvr_ctx* c) {
     return RIHVR_OK;
 }
 
-// the residual norms are reduced over spectra FFT(r) / N: |r|^2 = N sum |FFT(r) / N|^2
-void scale_resid_norms(rihvr_ctx* c) {
-    c->h_scal[SL_RESID_A] *= (double)c->N;
-    c->h_scal[SL_RESID_M] *= (double)c->N;
+static_assert(SL_COUNT == 16 && SL_SEQ == SL_COUNT - 1, "the context's blocks of scalars");
+
+// A block of scalars as the host works with it.  The residual norms are reduced over spectra
+// FFT(r) / N: |r|^2 = N sum |FFT(r) / N|^2.
+void take_scalars(rihvr_ctx* c, const double* block) {
+    std::memcpy(c->sc, block, sizeof(c->sc));
+    c->sc[SL_RESID_A] *= (double)c->N;
+    c->sc[SL_RESID_M] *= (double)c->N;
+}
+
+// A block of scalars from the device, in stream order
+rihvr_status copy_scalars(rihvr_ctx* c, const double* from) {
+    RIHVR_HIP(hipMemcpyAsync(c->h_scal + SL_COUNT, from, SL_COUNT * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    RIHVR_HIP(hipStreamSynchronize(c->stream));
+    take_scalars(c, c->h_scal + SL_COUNT);
+    return RIHVR_OK;
 }
 
 rihvr_status fetch_scalars(rihvr_ctx* c) {
-    RIHVR_HIP(hipMemcpyAsync(c->h_scal, c->scal, SL_COUNT * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    RIHVR_HIP(hipStreamSynchronize(c->stream));
-    scale_resid_norms(c);
+    RIHVR_TRY(copy_scalars(c, c->scal));
     return resolve_timing(c);
 }
 
-// The scalars as A's reduction (forward_finish) wrote them to h_scal, waited for by an event
-// recorded after it, so that work queued later keeps the device busy.  The next A writes h_scal
-// again: it is queued only after the host has read it.
+// The scalars as A's reduction (forward_finish) published them, waited for by an event recorded after
+// it, so that work queued later keeps the device busy.  The host decides the solve's path from them
+// (backtracks, the step, restarts) while the device goes by its own copy, so a block of another
+// iteration would not show as an error but as a wrong volume: the block's number is compared, and one
+// that is late is counted and taken by a copy after everything queued.
 rihvr_status wait_scalars(rihvr_ctx* c) {
     RIHVR_HIP(hipEventSynchronize(c->ev_scal));
-    scale_resid_norms(c);
+    if (c->test_late && c->ss.iters < 64) {
+        double now[SL_COUNT];
+        std::memcpy(now, c->h_scal, sizeof(now));
+        if ((c->test_late >> c->ss.iters) & 1ull) std::memcpy(c->h_scal, c->test_prev, sizeof(now));
+        std::memcpy(c->test_prev, now, sizeof(now));
+    }
+    double seq;
+    __atomic_load(c->h_scal + SL_SEQ, &seq, __ATOMIC_ACQUIRE);
+    if (seq == c->published) {
+        take_scalars(c, c->h_scal);
+    } else {
+        ++c->counters.late_scalars;
+        RIHVR_TRY(copy_scalars(c, c->scal_pub));
+        if (c->sc[SL_SEQ] != c->published) return RIHVR_E_DEVICE;
+    }
     return resolve_timing(c);
 }
 
@@ -380,9 +414,11 @@ rihvr_status forward_finish(rihvr_ctx* c, float2* est) {
         return holo_spec(c->spart, c->nparts, c->N, c->W, c->H, c->bspec, est, c->partial_holo, c->stream);
     }));
     RIHVR_TRY(timed(c, K_REDUCE, [&] {
+        const Publish pub{c->scal, c->scal_pub, c->h_scal, SL_COUNT};
         return reduce_partials(c->partial_holo, holo_spec_num_blocks(c->W, c->H), 1, c->red_work, c->scal + SL_RESID_A,
-                               c->stream, c->scal, c->h_scal, SL_COUNT);
+                               c->stream, &pub);
     }));
+    c->published += 1;
     return RIHVR_OK;
 }
 
@@ -611,7 +647,7 @@ void release(rihvr_ctx* c) {
     void* ptrs[] = {c->G, c->G_alt, c->T, c->tvbuf, c->meas, c->hE, c->hC, c->hP, c->hX, c->resid, c->rhat, c->htmp, c->bspec,
                     c->hspat, c->spart, c->kappa,
                     c->zlist, c->phase, c->phase_fwd, c->twfW, c->twiW, c->twfH, c->twiH, c->partial, c->partial_holo, c->scal,
-                    c->red_work, c->dflag};
+                    c->scal_pub, c->red_work, c->dflag};
     for (void* q : ptrs) (void)hipFree(q);
     for (auto& p : c->tm.pending) { (void)hipEventDestroy(p.a); (void)hipEventDestroy(p.b); }
     for (hipEvent_t e : c->tm.pool) (void)hipEventDestroy(e);
@@ -720,6 +756,7 @@ rihvr_status create_impl(const rihvr_params* params, const rihvr_schedule* sch, 
     c->n_groups = (c->Nz + c->pipe_planes - 1) / c->pipe_planes;
     if (const char* e = std::getenv("RIHVR_GROUP_ONE_STREAM")) c->groups_one_stream = std::atoi(e) != 0;
     if (const char* e = std::getenv("RIHVR_TEST_BACKTRACKS")) c->test_backtracks = std::strtoull(e, nullptr, 0);
+    if (const char* e = std::getenv("RIHVR_TEST_LATE_SCALARS")) c->test_late = std::strtoull(e, nullptr, 0);
     c->ev_adj.assign(c->n_groups, nullptr);
     for (hipEvent_t& e : c->ev_adj) RIHVR_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     for (auto& b : c->Yb) RIHVR_TRY(dalloc(&b, c->V));
@@ -763,11 +800,13 @@ rihvr_status create_impl(const rihvr_params* params, const rihvr_schedule* sch, 
     if (c->rad_h) c->holo_rows = std::max<long>(c->holo_rows, gen_cols_blocks(c->H, c->W));
     RIHVR_TRY(dalloc(&c->partial_holo, c->holo_rows));
     RIHVR_TRY(dalloc(&c->scal, SL_COUNT));
+    RIHVR_HIP(hipMemsetAsync(c->scal, 0, SL_COUNT * sizeof(double), c->stream));
+    RIHVR_TRY(dalloc(&c->scal_pub, SL_COUNT));
     RIHVR_TRY(dalloc(&c->red_work, (size_t)kReduceBlocks * PS_COUNT));
     RIHVR_TRY(dalloc(&c->dflag, 4));
     RIHVR_TRY(dalloc(&c->d_smom, 1));
     RIHVR_TRY(dalloc(&c->d_step, 1));
-    RIHVR_HIP(hipHostMalloc((void**)&c->h_scal, SL_COUNT * sizeof(double), hipHostMallocDefault));
+    RIHVR_HIP(hipHostMalloc((void**)&c->h_scal, 2 * SL_COUNT * sizeof(double), hipHostMallocDefault));
 
     // kappa table, plane list and per-plane phase factors, computed on the host
     // exactly as the reference does (sparse_compressive_holo.cu:38-56;
@@ -890,14 +929,15 @@ rihvr_status begin_impl(rihvr_ctx* c, const float* holo, int holo_loc, const flo
         }));
     }
     RIHVR_TRY(fetch_scalars(c));
+    c->published = c->sc[SL_SEQ];  // (a call that failed may have counted a block that never ran)
     int hflag = 0;
-    std::memcpy(&hflag, c->h_scal + SL_FLAG, sizeof(int));
+    std::memcpy(&hflag, c->sc + SL_FLAG, sizeof(int));
     if (hflag) return RIHVR_E_INVALID_DATA;
     if (warm) {
-        l1 = c->h_scal[SL_PROX + PS_L1X0];
-        tv = c->h_scal[SL_PROX + PS_TVX0];
+        l1 = c->sc[SL_PROX + PS_L1X0];
+        tv = c->sc[SL_PROX + PS_TVX0];
     }
-    c->ss.prev_summag = c->h_scal[SL_RESID_A];
+    c->ss.prev_summag = c->sc[SL_RESID_A];
     c->ss.f_initial = objective(c, c->ss.mode, c->ss.prev_summag, l1, tv);
     if (f_initial) *f_initial = c->ss.f_initial;
     // the residual's spectrum; the gradient's planes are formed with the first prox
@@ -928,7 +968,7 @@ rihvr_status momentum_objective(rihvr_ctx* c, double summag, double* f) {
                                c->red_work, c->scal + SL_PROX, c->stream);
     }));
     RIHVR_TRY(fetch_scalars(c));
-    *f = objective(c, c->ss.mode, summag, c->h_scal[SL_PROX + PS_L1X0], c->h_scal[SL_PROX + PS_TVX0]);
+    *f = objective(c, c->ss.mode, summag, c->sc[SL_PROX + PS_L1X0], c->sc[SL_PROX + PS_TVX0]);
     return RIHVR_OK;
 }
 
@@ -1027,7 +1067,10 @@ rihvr_status iterate_impl(rihvr_ctx* c, int n_it, rihvr_stats* st, bool last_f_b
                             RIHVR_TRY(apply_prox(c, mode, Y0, YM, s.s_mom, c->G, s.t, Yn, c->d_smom, true, form));
                             return apply_forward(c, Yn, c->hX);
                         },
-                        [&] { return apply_prox(c, mode, Y0, YM, s.s_mom, c->G, s.t, Yn, c->d_smom, false, form); }));
+                        [&] {
+                            c->published += 1;
+                            return apply_prox(c, mode, Y0, YM, s.s_mom, c->G, s.t, Yn, c->d_smom, false, form);
+                        }));
                 } else {
                     RIHVR_TRY(apply_prox(c, mode, Y0, YM, s.s_mom, c->G, s.t, Yn, nullptr, true, form));
                     RIHVR_TRY(apply_forward(c, Yn, c->hX));
@@ -1077,7 +1120,7 @@ rihvr_status iterate_impl(rihvr_ctx* c, int n_it, rihvr_stats* st, bool last_f_b
             } else {
                 RIHVR_TRY(fetch_scalars(c));
             }
-            const double* sc = c->h_scal;
+            const double* sc = c->sc;
             if (bt == 0 && s.iters > 0) {
                 // residual norm at the previous momentum point (:545-549), and the
                 // objective there from this prox's x0 reductions
@@ -1128,10 +1171,15 @@ rihvr_status iterate_impl(rihvr_ctx* c, int n_it, rihvr_stats* st, bool last_f_b
             break;
         }
         if (i == n_it) break;  // stopped at the objective target
-        s.nnz_y = c->h_scal[SL_PROX + PS_NNZY];
-        if (form == ProxForm::scan && c->h_scal[SL_PROX + PS_SKIPPED] < kScanPays * (double)c->prox_strip_rows)
+        s.nnz_y = c->sc[SL_PROX + PS_NNZY];
+        if (c->dense_ok && mode == RIHVR_MODE_FASTA_FUSED_LASSO_2D) {
+            rihvr_counters& n = c->counters;
+            ++(form == ProxForm::dense ? n.prox_dense : form == ProxForm::scan ? n.prox_scan : n.prox_rows);
+            if (form == ProxForm::scan) n.scan_skipped += (int64_t)c->sc[SL_PROX + PS_SKIPPED];
+        }
+        if (form == ProxForm::scan && c->sc[SL_PROX + PS_SKIPPED] < kScanPays * (double)c->prox_strip_rows)
             s.scan_below = s.nnz_y / 2;
-        const double rs = c->h_scal[SL_PROX + PS_RESTART];
+        const double rs = c->sc[SL_PROX + PS_RESTART];
         const bool restart = rs > 0;  // :4481
         if (restart) alpha0 = 1;
         s.alpha1 = (1.0 + std::sqrt(1.0 + 4.0 * alpha0 * alpha0)) / 2.0;  // :476
@@ -1181,12 +1229,12 @@ rihvr_status iterate_impl(rihvr_ctx* c, int n_it, rihvr_stats* st, bool last_f_b
         st->f_initial = s.f_initial;
         if (n_it > 0 && !last_f_by_finish && (st->f || st->f_resid || st->sparsity_it)) {
             RIHVR_TRY(fetch_scalars(c));
-            const double summag = c->h_scal[SL_RESID_M];
+            const double summag = c->sc[SL_RESID_M];
             double f = 0;
             RIHVR_TRY(momentum_objective(c, summag, &f));
             if (st->f) st->f[n_it - 1] = f;
             if (st->f_resid) st->f_resid[n_it - 1] = 0.5 * summag;
-            if (st->sparsity_it) st->sparsity_it[n_it - 1] = c->h_scal[SL_PROX + PS_NNZX0] / (double)c->V;
+            if (st->sparsity_it) st->sparsity_it[n_it - 1] = c->sc[SL_PROX + PS_NNZX0] / (double)c->V;
         }
     }
     return RIHVR_OK;
@@ -1208,7 +1256,7 @@ rihvr_status finish_impl(rihvr_ctx* c, rihvr_stats* st, int last_index) {
                                c->scal + SL_PROX, c->stream);
     }));
     RIHVR_TRY(fetch_scalars(c));
-    const double* sc = c->h_scal;
+    const double* sc = c->sc;
     const double summag = s.iters > 0 ? sc[SL_RESID_M] : s.prev_summag;
     const double f_last = objective(c, s.mode, summag, sc[SL_PROX + PS_L1X0], sc[SL_PROX + PS_TVX0]);
     c->out = outb;
@@ -1339,7 +1387,7 @@ rihvr_status learned_impl(rihvr_ctx* c, rihvr_net* net, const float* holo, int h
     RIHVR_HIP(holo_residual(c->bspec, c->hC, c->htmp, c->N, c->partial_holo, c->stream));
     RIHVR_TRY(reduce_partials_on(c, c->partial_holo, holo_num_blocks(c->N), 1, c->scal + SL_RESID_M));
     RIHVR_TRY(fetch_scalars(c));
-    st.f_zero = 0.5 * c->h_scal[SL_RESID_M];
+    st.f_zero = 0.5 * c->sc[SL_RESID_M];
     // objective and data residual of a start volume X
     // (map: X's valid line-occupancy map, or NULL)
     auto volume_objective = [&](const float2* X, const uint64_t* map, double* resid, double* f) -> rihvr_status {
@@ -1351,8 +1399,8 @@ rihvr_status learned_impl(rihvr_ctx* c, rihvr_net* net, const float* holo, int h
         RIHVR_TRY(reduce_partials_on(c, c->partial, momentum_out_num_blocks(c->W, c->H, c->Nz), PS_COUNT,
                                      c->scal + SL_PROX));
         RIHVR_TRY(fetch_scalars(c));
-        *resid = 0.5 * c->h_scal[SL_RESID_A];
-        *f = objective(c, mode, c->h_scal[SL_RESID_A], c->h_scal[SL_PROX + PS_L1X0], c->h_scal[SL_PROX + PS_TVX0]);
+        *resid = 0.5 * c->sc[SL_RESID_A];
+        *f = objective(c, mode, c->sc[SL_RESID_A], c->sc[SL_PROX + PS_L1X0], c->sc[SL_PROX + PS_TVX0]);
         return RIHVR_OK;
     };
     // The network's output is dense (every voxel holds a small value), which the objective's L1
@@ -1427,7 +1475,7 @@ rihvr_status volume_norm2(rihvr_ctx* c, const float2* v, double* out) {
     RIHVR_HIP(norm2_partials(v, c->V, nb, c->partial, c->stream));
     RIHVR_TRY(reduce_partials_on(c, c->partial, nb, 1, c->scal + SL_RESID_M));
     RIHVR_TRY(fetch_scalars(c));
-    *out = c->h_scal[SL_RESID_M];
+    *out = c->sc[SL_RESID_M];
     return RIHVR_OK;
 }
 
@@ -1803,6 +1851,13 @@ rihvr_status rihvr_get_timing(rihvr_ctx* ctx, rihvr_kernel_time* out, int32_t ca
         out[k].launches = ctx->tm.launches[k];
         out[k].total_ms = ctx->tm.total_ms[k];
     }
+    return RIHVR_OK;
+}
+
+rihvr_status rihvr_get_counters(const rihvr_ctx* ctx, rihvr_counters* out) {
+    if (!ctx || !out) return RIHVR_E_INVALID_ARGUMENT;
+    *out = ctx->counters;
+    out->graphs = (int64_t)(ctx->gcache[0].size() + ctx->gcache[1].size());
     return RIHVR_OK;
 }
 
