@@ -135,10 +135,19 @@ __global__ void __launch_bounds__(RowCfg<L>::THREADS) k_rows(RowArgs a) {
         // The plane's strips as a wave-uniform mask (every wave loads the same bytes); a plane
         // without any strip adds zeros to the accumulators (never -0: they start at +0), so it
         // is skipped; absent strips are read as zeros.  The same for every wave: no barrier is
-        // skipped by part of the workgroup.
+        // skipped by part of the workgroup.  The last wave may have fewer lanes than a row has
+        // strips (896: 32 lanes, 56 strips), so where it does 32 lanes take two strips each.
+        constexpr int kLastLanes = C::THREADS % 64 ? C::THREADS % 64 : 64;
+        static_assert(NS <= kLastLanes || kLastLanes >= 32, "every wave sees every strip");
         auto plane_mask = [&](int z) -> uint64_t {
             const uint8_t* sm = a.smap + (size_t)z * NS;
-            return __ballot(lane < NS && sm[lane < NS ? lane : 0] != 0);
+            auto strips = [&](int s, bool take) -> uint64_t {
+                return __ballot(take && s < NS && sm[s < NS ? s : 0] != 0);
+            };
+            if constexpr (NS <= kLastLanes)
+                return strips(lane, true);
+            else
+                return strips(lane, lane < 32) | (strips(lane + 32, lane < 32) << 32);
         };
         if constexpr (!row_regs_fast<L>()) {
             for (int z = z0; z < z1; ++z) {
