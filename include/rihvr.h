@@ -170,7 +170,8 @@ rihvr_status rihvr_reconstruct_batch(rihvr_ctx* ctx, const float* holos, int hol
  * that change speed but not the mathematics (the sums' order changes with them, so results
  * agree to rounding across schedules and bit for bit within one). */
 typedef struct rihvr_schedule {
-    int32_t fft_path;    /* 0: the fixed-length FFT kernels where the size has them, 1: run-time plans */
+    int32_t fft_path;    /* 0: the fixed-length FFT kernels along each axis whose length has them (run-time
+                            plans along the other), 1: run-time plans along both */
     int32_t max_radix;   /* largest radix of the run-time plans: 16, 8 or 4 */
     int32_t zchunk_fwd;  /* planes per partial spectrum of A */
     int32_t zchunk_adj;  /* planes per workgroup of A^T's first pass */

@@ -132,7 +132,8 @@ struct rihvr_ctx {
     // FFTs of lengths outside the fixed-length kernels' set (or all, by the schedule) run with
     // run-time plans (fft_generic.hip): the plans' largest radix along x and y, 0 for a fixed plan
     int rad_w = 0, rad_h = 0;
-    int gen_radix = 16;  // the schedule's choice
+    int gen_radix = 16;      // the schedule's choice
+    bool force_gen = false;  // run-time plans asked for along both axes
     float2* tvbuf = nullptr;                      // 4 volumes for mode 7 with n_tv above the fused prox's limit
     float2* out = nullptr;                        // points at the returned volume
     // holograms
@@ -717,13 +718,12 @@ rihvr_status create_impl(const rihvr_params* params, const rihvr_schedule* sch, 
     // workgroup, where its fields are 0.  Without one, split_planes gives small problems more and
     // shorter chunks.
     int zc = 32, za = 8, prow = -1;
-    bool force_gen = false;
     if (sch) {
         if (sch->zchunk_fwd > 0) zc = sch->zchunk_fwd;
         if (sch->zchunk_adj > 0) za = sch->zchunk_adj;
         if (sch->prox_rows > 0) prow = sch->prox_rows;
         if (sch->max_radix > 0) c->gen_radix = sch->max_radix;
-        force_gen = sch->fft_path == 1;
+        c->force_gen = sch->fft_path == 1;
         c->graphs = sch->graphs != 0;
     } else {
         default_chunks(c->W, c->H, c->Nz, &zc, &za);
@@ -748,8 +748,8 @@ rihvr_status create_impl(const rihvr_params* params, const rihvr_schedule* sch, 
     pp = ((pp + 15) / 16) * 16;
     c->pipe_planes = std::min(c->Nz, std::max(16, pp));
     if (c->pipe_planes % c->zchunk_fwd || c->pipe_planes % c->zchunk_adj) c->pipe_planes = c->Nz;
-    c->rad_w = force_gen || !fft_length_supported(c->W) ? c->gen_radix : 0;
-    c->rad_h = force_gen || !fft_length_supported(c->H) ? c->gen_radix : 0;
+    c->rad_w = c->force_gen || !fft_length_supported(c->W) ? c->gen_radix : 0;
+    c->rad_h = c->force_gen || !fft_length_supported(c->H) ? c->gen_radix : 0;
     const bool tv_general = params->mode == RIHVR_MODE_FASTA_FUSED_LASSO_2D &&
                             !prox_fl2d_supported(params->num_tv_iterations);
     if (tv_general) c->pipe_planes = c->Nz;  // the plane-group schedule needs the fused prox
@@ -1511,9 +1511,11 @@ rihvr_status lipschitz_impl(rihvr_ctx* c, int seed, int iterations, double* L) {
     return RIHVR_OK;
 }
 
+// A context made from it takes the same kernels.  (Where one axis has a fixed plan and the other not,
+// path 0 is the mix of both and path 1 run-time plans along both.)
 rihvr_schedule schedule_of(const rihvr_ctx* c) {
     rihvr_schedule s{};
-    s.fft_path = c->rad_w || c->rad_h ? 1 : 0;
+    s.fft_path = c->rad_w && c->rad_h ? 1 : 0;
     s.max_radix = c->gen_radix;
     s.zchunk_fwd = c->zchunk_fwd;
     s.zchunk_adj = c->zchunk_adj;
@@ -1596,11 +1598,11 @@ rihvr_status autotune_impl(const rihvr_params* p, const float* holo, int holo_lo
     cur.max_radix = 16;
     default_chunks(p->width, p->height, p->num_planes, &cur.zchunk_fwd, &cur.zchunk_adj);
     cur.graphs = 1;
-    const bool fixed = fft_length_supported(p->width) && fft_length_supported(p->height);
-    if (!fixed) cur.fft_path = 1;
+    const bool fixed_w = fft_length_supported(p->width), fixed_h = fft_length_supported(p->height);
+    if (!fixed_w && !fixed_h) cur.fft_path = 1;
     RIHVR_TRY(measure(cur));
-    // a candidate that does not fit in memory (the run-time plans' transposed planes take one more
-    // volume) is skipped; any other error ends the search
+    // a candidate that does not fit in memory (more partial spectra) is skipped; any other error ends
+    // the search
     auto try_set = [&](std::vector<rihvr_schedule> cands) -> rihvr_status {
         for (rihvr_schedule s : cands) {
             if (same(s, cur)) continue;
@@ -1612,12 +1614,15 @@ rihvr_status autotune_impl(const rihvr_params* p, const float* holo, int holo_lo
         return RIHVR_OK;
     };
     std::vector<rihvr_schedule> v;
-    for (int r : {16, 8, 4}) {
-        rihvr_schedule s = cur;
-        s.fft_path = 1;
-        s.max_radix = r;
-        v.push_back(s);
-    }
+    for (int path : {0, 1})
+        for (int r : {16, 8, 4}) {
+            // path 0 has run-time plans, and their radix, only beside one fixed length
+            if (path == 0 && fixed_w == fixed_h) continue;
+            rihvr_schedule s = cur;
+            s.fft_path = path;
+            s.max_radix = r;
+            v.push_back(s);
+        }
     RIHVR_TRY(try_set(v));
     const rihvr_schedule base = cur;
     v.clear();
