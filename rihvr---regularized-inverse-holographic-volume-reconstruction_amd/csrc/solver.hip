@@ -714,6 +714,13 @@ rihvr_status create_impl(const rihvr_params* params, const rihvr_schedule* sch, 
     RIHVR_HIP(hipStreamCreateWithFlags(&c->aux, hipStreamNonBlocking));
     RIHVR_HIP(hipEventCreateWithFlags(&c->ev_rhat, hipEventDisableTiming));
     RIHVR_HIP(hipEventCreateWithFlags(&c->ev_scal, hipEventDisableTiming));
+    // pipeline groups: one group (everything on the main stream) unless RIHVR_PIPE_PLANES
+    // asks for groups of that many planes (rounded up to a multiple of 16).  Measured at
+    // 1024^2 x 128 on MI355X the two-stream overlap loses (groups of 32: 287 iter/s,
+    // 64: 308, one stream: 316): the prox and the column FFTs each fill the CUs' LDS, so
+    // they time-share CUs instead of co-issuing
+    int group = 0;
+    if (const char* e = std::getenv("RIHVR_PIPE_PLANES")) group = (std::max(0, std::atoi(e)) + 15) / 16 * 16;
     // With a schedule: A's partial spectra over 32 planes, A^T's row pass over 8 planes per
     // workgroup, where its fields are 0.  Without one, split_planes gives small problems more and
     // shorter chunks.
@@ -727,6 +734,10 @@ rihvr_status create_impl(const rihvr_params* params, const rihvr_schedule* sch, 
         c->graphs = sch->graphs != 0;
     } else {
         default_chunks(c->W, c->H, c->Nz, &zc, &za);
+        if (group > 0 && group < c->Nz) {  // groups hold whole chunks
+            while (group % zc) --zc;
+            while (group % za) --za;
+        }
         if (const char* e = std::getenv("RIHVR_ZCHUNK")) zc = std::max(1, std::atoi(e));
         if (const char* e = std::getenv("RIHVR_ZCHUNK_ADJ")) za = std::max(1, std::atoi(e));
         if (const char* e = std::getenv("RIHVR_PROX_ROWS")) prow = std::max(0, std::atoi(e));
@@ -738,15 +749,7 @@ rihvr_status create_impl(const rihvr_params* params, const rihvr_schedule* sch, 
     c->zchunk_fwd = std::min(c->Nz, zc);
     c->nparts = (c->Nz + c->zchunk_fwd - 1) / c->zchunk_fwd;
     c->zchunk_adj = std::min(c->Nz, za);
-    // pipeline groups: one group (everything on the main stream) unless RIHVR_PIPE_PLANES
-    // asks for groups of that many planes (rounded up to a multiple of 16).  Measured at
-    // 1024^2 x 128 on MI355X the two-stream overlap loses (groups of 32: 287 iter/s,
-    // 64: 308, one stream: 316): the prox and the column FFTs each fill the CUs' LDS, so
-    // they time-share CUs instead of co-issuing
-    int pp = c->Nz;
-    if (const char* e = std::getenv("RIHVR_PIPE_PLANES")) pp = std::atoi(e) > 0 ? std::atoi(e) : c->Nz;
-    pp = ((pp + 15) / 16) * 16;
-    c->pipe_planes = std::min(c->Nz, std::max(16, pp));
+    c->pipe_planes = group > 0 ? std::min(c->Nz, group) : c->Nz;
     if (c->pipe_planes % c->zchunk_fwd || c->pipe_planes % c->zchunk_adj) c->pipe_planes = c->Nz;
     c->rad_w = c->force_gen || !fft_length_supported(c->W) ? c->gen_radix : 0;
     c->rad_h = c->force_gen || !fft_length_supported(c->H) ? c->gen_radix : 0;
