@@ -254,16 +254,22 @@ rihvr_status copy_out(rihvr_ctx* c, float* dst, const float2* src, int loc, size
     return RIHVR_OK;
 }
 
-// Whether the context's kernels can work on caller memory in place: device memory of its GPU,
-// aligned for complex64.  Anything else that a copy accepts is copied.
-bool in_place(const rihvr_ctx* c, const void* p, int loc) {
+// Whether the context's kernels can work on `count` complex64 values of caller memory in place: device
+// memory of its GPU, aligned for complex64, within one allocation.  Anything else goes through a copy,
+// which takes what it can read or write and refuses the rest (an allocation that is too small, which a
+// kernel would run past).
+bool in_place(const rihvr_ctx* c, const void* p, int loc, size_t count) {
     if (loc != RIHVR_DEVICE || (uintptr_t)p % sizeof(float2)) return false;
     hipPointerAttribute_t a{};
-    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    hipDeviceptr_t base{};
+    size_t size = 0;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess || a.type != hipMemoryTypeDevice || a.device != c->device ||
+        hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)p) != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
-    return a.type == hipMemoryTypeDevice && a.device == c->device;
+    const size_t at = (size_t)((const char*)p - (const char*)base);
+    return at <= size && count * sizeof(float2) <= size - at;
 }
 
 // Launches through `launch` (returns hipError_t) on stream `st`, bracketed by events
@@ -1909,7 +1915,7 @@ rihvr_status rihvr_forward(rihvr_ctx* ctx, const float* volume, int vol_loc, flo
     ctx->have_result = false;
     ctx->ss.active = false;
     const float2* v = (const float2*)volume;
-    if (!in_place(ctx, volume, vol_loc)) {
+    if (!in_place(ctx, volume, vol_loc, ctx->V)) {
         ctx->occ_valid[0] = false;
         RIHVR_TRY(copy_in(ctx, ctx->Yb[0], volume, vol_loc, ctx->V));
         v = ctx->Yb[0];
@@ -1928,7 +1934,7 @@ rihvr_status rihvr_adjoint(rihvr_ctx* ctx, const float* holo, int holo_loc, floa
     RIHVR_TRY(copy_in(ctx, ctx->resid, holo, holo_loc, ctx->N));
     // the last pass writes a device volume where the caller wants it (the copy was 210 of 830 us at
     // 2048^2 x 16)
-    if (in_place(ctx, volume_out, vol_loc)) {
+    if (in_place(ctx, volume_out, vol_loc, ctx->V)) {
         RIHVR_TRY(apply_adjoint(ctx, ctx->resid, (float2*)volume_out));
         RIHVR_HIP(hipStreamSynchronize(ctx->stream));
         return RIHVR_OK;
