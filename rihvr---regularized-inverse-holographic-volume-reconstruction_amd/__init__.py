@@ -217,6 +217,21 @@ class Object(ctypes.Structure):
                     max_value=self.max_value, mean_value=self.mean_value, num_voxels=self.num_voxels,
                     label=self.label, bounds=list(self.bounds))
 
+    @staticmethod
+    def as_dicts(arr, n) -> list:
+        """[arr[i].as_dict() for i in range(n)].  From 2 objects on all fields at once through numpy: us
+        for 0, 1, 2, 5, 16 and 500 objects 1.4, 1.9, 2.1, 3.0, 6.0 and 155, one by one 0.2, 1.5, 2.7, 6.2,
+        19 and 597."""
+        if n < 2:
+            return [arr[i].as_dict() for i in range(n)]
+        cols = np.frombuffer(arr, _OBJECT_DTYPE, n)
+        return [dict(centroid=c, weighted_centroid=w, max_value=hi, mean_value=mean, num_voxels=size, label=label,
+                     bounds=box)
+                for c, w, hi, mean, size, label, box in zip(*(cols[k].tolist() for k, _ in Object._fields_))]
+
+
+_OBJECT_DTYPE = np.dtype(Object)
+
 
 class LearnedStats(ctypes.Structure):
     """Mirror of ``rihvr_learned_stats`` (include/rihvr.h)."""
@@ -1213,11 +1228,7 @@ class ObjectCloud:
         got = ctypes.c_int64()
         _check(lib().rihvr_segmentation_objects(self._seg._h, arr, n, ctypes.byref(got)),
                "rihvr_segmentation_objects")
-        # all fields at once through numpy (an object's conversion by ctypes takes 3 us)
-        cols = np.frombuffer(arr, np.dtype(Object), n)
-        c, w, hi, mean, size, label, box = (np.ascontiguousarray(cols[k]).tolist() for k, _ in Object._fields_)
-        return [dict(centroid=c[i], weighted_centroid=w[i], max_value=hi[i], mean_value=mean[i], num_voxels=size[i],
-                     label=label[i], bounds=box[i]) for i in range(n)]
+        return Object.as_dicts(arr, n)
 
     def blobSizeFilter(self, min_size) -> int:
         removed = ctypes.c_int64()
