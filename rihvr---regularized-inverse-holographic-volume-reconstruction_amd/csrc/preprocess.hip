@@ -85,7 +85,9 @@ struct Geometry {
 // contiguous; that needs an even ow and a 16-byte aligned output.  The holograms are written past
 // the caches: they are eight times the frames' bytes and read by a later call.  What bounds it is that
 // stream: 100 frames of 1024^2 take 183 us a call (5.2 TB/s, a copy reaches 5.14), 281 before with 32 bytes a
-// thread in two ordinary stores.
+// thread in two ordinary stores.  Small outputs, which the caches would hold, gain less or nothing (us,
+// ordinary stores against these: 10 frames of 1024^2 43.1, 41.5; 40 of 512^2 40.3, 37.2; 32 of 166^2
+// 25.9, 26.8), so there is no rule by size.
 // Every pixel's loads are issued unconditionally (pixel 0 of the frame stands in for a pixel outside
 // the crop or the image) so that they overlap; the select afterwards keeps zero for those pixels.
 template <typename T, int PIX>
@@ -182,16 +184,15 @@ rihvr_status run_with(const T* frames, const float* bg, const Geometry& g, int n
     }
     // frames in launches of at most kMaxGridYZ (the grid's y and z limit)
     const bool wide = g.ow % 2 == 0 && (size_t)out_dev % 16 == 0;
-    const int pix = wide ? kPix : 1;
+    // a row of at most 2 kThreads pixels has no second pair for a thread (100 frames of 512^2 58.3 us, with
+    // the second pair's loads and no store for them 61.5)
+    const int pix = !wide ? 1 : g.ow <= 2 * kThreads ? 2 : kPix;
+    const auto write = pix == 1 ? k_pre_write<T, 1> : pix == 2 ? k_pre_write<T, 2> : k_pre_write<T, kPix>;
     for (int f0 = 0; f0 < n; f0 += kMaxGridYZ) {
         const dim3 grid((unsigned)((g.ow + kThreads * pix - 1) / (kThreads * pix)), (unsigned)g.oh,
                         (unsigned)std::min(n - f0, kMaxGridYZ));
-        if (wide)
-            hipLaunchKernelGGL((k_pre_write<T, kPix>), grid, dim3(kThreads), 0, 0, frames, bg, g, f0, inv255,
-                               (const float*)inv_mean, (float2*)out_dev);
-        else
-            hipLaunchKernelGGL((k_pre_write<T, 1>), grid, dim3(kThreads), 0, 0, frames, bg, g, f0, inv255,
-                               (const float*)inv_mean, (float2*)out_dev);
+        hipLaunchKernelGGL(write, grid, dim3(kThreads), 0, 0, frames, bg, g, f0, inv255, (const float*)inv_mean,
+                           (float2*)out_dev);
     }
     PRE_HIP(hipGetLastError());
     PRE_HIP(hipDeviceSynchronize());
