@@ -15,6 +15,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <string>
 #include <vector>
 
 #include "../../include/rihvr.h"
@@ -193,7 +194,10 @@ struct rihvr_ctx {
     // first attempt of those iterations is rejected as if its ratio were above 1, so the
     // backtracking paths can be exercised; never set in normal use
     uint64_t test_backtracks = 0;
-    // the same for RIHVR_TEST_LATE_SCALARS: in those iterations the host finds the block published before
+    // RIHVR_TEST_PROX_FORM (rows, scan or dense): the form of every fused mode-7 prox, whatever the iterate
+    bool test_form = false;
+    ProxForm forced_form = ProxForm::rows;
+    // as RIHVR_TEST_BACKTRACKS for RIHVR_TEST_LATE_SCALARS: in those iterations the host finds the block published before
     uint64_t test_late = 0;
     double test_prev[16] = {};
     Timer tm;
@@ -765,6 +769,11 @@ rihvr_status create_impl(const rihvr_params* params, const rihvr_schedule* sch, 
     c->n_groups = (c->Nz + c->pipe_planes - 1) / c->pipe_planes;
     if (const char* e = std::getenv("RIHVR_GROUP_ONE_STREAM")) c->groups_one_stream = std::atoi(e) != 0;
     if (const char* e = std::getenv("RIHVR_TEST_BACKTRACKS")) c->test_backtracks = std::strtoull(e, nullptr, 0);
+    if (const char* e = std::getenv("RIHVR_TEST_PROX_FORM")) {
+        const std::string f = e;
+        c->test_form = f == "rows" || f == "scan" || f == "dense";
+        c->forced_form = f == "scan" ? ProxForm::scan : f == "dense" ? ProxForm::dense : ProxForm::rows;
+    }
     if (const char* e = std::getenv("RIHVR_TEST_LATE_SCALARS")) c->test_late = std::strtoull(e, nullptr, 0);
     c->ev_adj.assign(c->n_groups, nullptr);
     for (hipEvent_t& e : c->ev_adj) RIHVR_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
@@ -1053,6 +1062,7 @@ rihvr_status iterate_impl(rihvr_ctx* c, int n_it, rihvr_stats* st, bool last_f_b
         else if (c->dense_ok && s.nnz_y > 0 && s.nnz_y < std::min(s.scan_below, kScanFraction * (double)c->V) &&
                  c->prox_rows >= kScanRows)
             form = ProxForm::scan;
+        if (c->test_form && c->dense_ok) form = c->forced_form;
         for (;;) {
             const bool use_graph = ahead && c->graphs && !c->tm.on;
             if (!s.g_ready && mode == RIHVR_MODE_FASTA_FUSED_LASSO_2D && c->n_groups > 1) {
