@@ -175,7 +175,9 @@ typedef struct rihvr_schedule {
     int32_t max_radix;   /* largest radix of the run-time plans: 16, 8 or 4 */
     int32_t zchunk_fwd;  /* planes per partial spectrum of A */
     int32_t zchunk_adj;  /* planes per workgroup of A^T's first pass */
-    int32_t prox_rows;   /* output rows per wave of the fused mode-7 prox (0: the device rule) */
+    int32_t prox_rows;   /* output rows per wave of the fused mode-7 prox, in each of its forms.  0, and
+                            the number that the device rule gives (which a context reports): the rule,
+                            which the dense form has of its own */
     int32_t graphs;      /* 1: the queued iterations run as captured HIP graphs */
     double  ms_per_iteration;  /* measured by rihvr_autotune (else 0) */
 } rihvr_schedule;
@@ -277,6 +279,7 @@ typedef struct rihvr_counters {
     int64_t prox_dense;    /* ... and in its dense form */
     int64_t scan_skipped;  /* rows (of the waves' strips) that the scans skipped */
     int64_t graphs;        /* captured graphs held now */
+    int64_t dense_rows;    /* output rows per wave of the dense form (0: not in use or the default) */
 } rihvr_counters;
 rihvr_status rihvr_get_counters(const rihvr_ctx* ctx, rihvr_counters* out);
 

@@ -153,7 +153,7 @@ class Counters(ctypes.Structure):
     """Mirror of ``rihvr_counters`` (include/rihvr.h): what a context's solves did."""
 
     _fields_ = [(k, ctypes.c_int64) for k in ("late_scalars", "prox_rows", "prox_scan", "prox_dense", "scan_skipped",
-                                              "graphs")]
+                                              "graphs", "dense_rows")]
 
     def as_dict(self) -> dict:
         return {k: getattr(self, k) for k, _ in self._fields_}

@@ -30,6 +30,9 @@ namespace rihvr {
 constexpr int kDefaultRowChunk = 128;  // output rows per wave
 constexpr int kProxWaves = 4;    // waves per workgroup
 constexpr int kMinRowChunk = 4;  // fewest output rows per wave that a rule picks
+// most output rows per wave that the dense form's rule picks: a lane sums the line search's and the
+// objective's terms of its column in 32 bits over them
+constexpr int kMaxDenseRows = 256;
 constexpr int kMaxNtv = 10;
 
 struct ProxGeom {
@@ -836,13 +839,16 @@ template <int NTV> static int fl2d_blocks_per_cu() {
 }
 
 // Output rows per wave of least cost for `strips` strips of H rows: rounds of `slots` resident
-// waves, each (rows + 2 n_tv + 1) steps of a + b w us, and at least `least`, with w waves on a SIMD.
-static int cheapest_rows(long strips, int H, int n_tv, long slots, int cus, double a, double b, double least) {
+// waves, each (rows + 2 n_tv + 1) steps of a + b w us, and at least `least`, with w waves on a SIMD; at
+// most `most` rows.
+static int cheapest_rows(long strips, int H, int n_tv, long slots, int cus, double a, double b, double least,
+                         int most) {
     auto step = [&](long waves) { return std::max(least, a + b * (double)waves / (4.0 * cus)); };
     double best_cost = 0;
     int best_rc = 0;
     for (int nch = 1; nch <= H; ++nch) {
         const int rc = (H + nch - 1) / nch;
+        if (rc > most) continue;
         if (rc < kMinRowChunk && nch > 1) break;
         const long waves = strips * ((H + rc - 1) / rc);
         const double t = (double)(waves / slots) * step(slots) + (waves % slots ? step(waves % slots) : 0.0);
@@ -886,7 +892,7 @@ int prox_fl2d_auto_rows(int W, int H, int nz, int n_tv) {
     // 256^2 x 32 67 with 8 against 97 with 32, 512^2 x 20 115 with 24 against 125 with 32).
     const int nch_target = std::max(1, (H + 102) / 205);
     if ((long)nstrips * nch_target * nz >= 2 * slots) return (H + nch_target - 1) / nch_target;
-    return cheapest_rows((long)nstrips * nz, H, n_tv, slots, cus, 1.7, 0.35, 0.0);
+    return cheapest_rows((long)nstrips * nz, H, n_tv, slots, cus, 1.7, 0.35, 0.0, H);
 }
 
 hipError_t prox_fl2d(const ProxLaunch& a, hipStream_t s) {
@@ -967,7 +973,7 @@ int prox_fl2d_dense_auto_rows(int W, int H, int nz, int n_tv) {
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         return 0;
     return cheapest_rows((long)prox_geom(W, H, n_tv, H).nstrips * nz, H, n_tv, (long)nb * kProxWaves * cus, cus, 0.18,
-                         0.45, 0.65);
+                         0.45, 0.65, kMaxDenseRows);
 }
 
 // ----------------------------------------------------------------------------

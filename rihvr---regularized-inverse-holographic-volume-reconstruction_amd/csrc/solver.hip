@@ -1882,6 +1882,7 @@ rihvr_status rihvr_get_counters(const rihvr_ctx* ctx, rihvr_counters* out) {
     if (!ctx || !out) return RIHVR_E_INVALID_ARGUMENT;
     *out = ctx->counters;
     out->graphs = (int64_t)(ctx->gcache[0].size() + ctx->gcache[1].size());
+    out->dense_rows = ctx->dense_ok ? ctx->prox_rows_dense : 0;
     return RIHVR_OK;
 }
 
