@@ -202,15 +202,20 @@ hipError_t holo_spec(const float2* parts, int nparts, long stride, int W, int H,
 // out = f * in
 hipError_t holo_scale(const float2* in, float2* out, long n, float f, hipStream_t s);
 
-// A block of n scalars that a reduction hands to the host: src's last value is raised by 1 (the number
-// of blocks handed over), the block is copied to snap (device) and host (pinned), the last value of host
-// after the others have reached it.
+// A block of n scalars (at most 64) that a reduction hands to the host: src's last value is raised by 1
+// (the number of blocks handed over), the block is copied to snap (device) and host (pinned), and
+// host[n] receives its check word, the sum of check_word over its values' bits.
 struct Publish {
     double* src;
     double* snap;
     double* host;
     int n;
 };
+__host__ __device__ inline uint64_t check_word(uint64_t bits, int i) {
+    uint64_t h = (bits ^ (0x9e3779b97f4a7c15ull * (uint64_t)(i + 1))) * 0xbf58476d1ce4e5b9ull;
+    h = (h ^ (h >> 29)) * 0x94d049bb133111ebull;
+    return h ^ (h >> 32);
+}
 
 // sums rows of partial [nrows][ncols] into out[ncols] (fixed order: deterministic);
 // work holds kReduceBlocks * ncols doubles.  Then publishes a block, when given (it may include out).

@@ -1729,9 +1729,10 @@ __global__ void __launch_bounds__(kReduceThreads) k_reduce_rows(const double* __
 }
 
 // The sums of all columns by one workgroup, in a fixed order; then the block of scalars for the host
-// (memory that the device writes: the scalars reach the host with the sums, without a copy).  The
-// block's number goes last, once the other values are visible to the host: a reader that finds the
-// number it expects has that block whole, and any other is seen to be late.
+// (memory that the device writes: the scalars reach the host with the sums, without a copy).  A reader
+// knows by the block's number and its check word whether it has that block, whole; the stores are not
+// ordered by a fence (50 iterations at 256^2 x 32 take 6.29 ms; 6.45 with a fence to the device
+// before them, 6.62 with one to the host before the number).
 constexpr int kReduceOneThreads = 1024;
 __global__ void __launch_bounds__(kReduceOneThreads)
 k_reduce_one(const double* __restrict__ partial, int nrows, int ncols, double* out, Publish pub) {
@@ -1758,19 +1759,20 @@ k_reduce_one(const double* __restrict__ partial, int nrows, int ncols, double* o
         out[threadIdx.x] = r;
     }
     if (!pub.host) return;
-    __threadfence();
-    __syncthreads();
-    const int i = threadIdx.x, last = pub.n - 1;
-    double v = 0.0;
-    if (i <= last) {
-        v = pub.src[i];
-        if (i == last) pub.src[i] = v += 1.0;
+    __syncthreads();  // out may be part of the block
+    const int i = threadIdx.x;
+    if (i >= 64) return;
+    unsigned long long check = 0;
+    if (i < pub.n) {
+        double v = pub.src[i];
+        if (i == pub.n - 1) pub.src[i] = v += 1.0;
         pub.snap[i] = v;
-        if (i < last) pub.host[i] = v;
+        pub.host[i] = v;
+        check = check_word((uint64_t)__double_as_longlong(v), i);
     }
-    __threadfence_system();
-    __syncthreads();
-    if (i == last) __hip_atomic_store(&pub.host[i], v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) check += __shfl_xor(check, off, 64);
+    if (i == 0) pub.host[pub.n] = __longlong_as_double((long long)check);
 }
 
 // One workgroup takes up to this many rows by itself: a launch less, which is what a reduction
@@ -1780,7 +1782,7 @@ constexpr int kReduceOneRows = 4096;
 
 hipError_t reduce_partials(const double* partial, int nrows, int ncols, double* work, double* out, hipStream_t s,
                            const Publish* pub) {
-    if (ncols < 1 || ncols > PS_COUNT || nrows < 0 || (pub && (pub->n < 1 || pub->n > kReduceOneThreads)))
+    if (ncols < 1 || ncols > PS_COUNT || nrows < 0 || (pub && (pub->n < 1 || pub->n > 64)))
         return hipErrorInvalidValue;
     if (nrows > kReduceOneRows) {
         const int rpb = (nrows + kReduceBlocks - 1) / kReduceBlocks;

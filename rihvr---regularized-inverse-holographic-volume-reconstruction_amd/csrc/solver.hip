@@ -160,7 +160,8 @@ struct rihvr_ctx {
     double* scal = nullptr;
     double* red_work = nullptr;  // first-pass sums of reduce_partials
     double* scal_pub = nullptr;  // the block of scalars that A's last reduction published
-    // pinned: the published block as the device writes it, then the target of stream-ordered copies
+    // pinned: the published block and its check word as the device writes them (kBlock values), then the
+    // target of stream-ordered copies
     double* h_scal = nullptr;
     double sc[16] = {};          // the scalars the host works with
     double published = 0;        // blocks published by the work queued so far
@@ -199,7 +200,7 @@ struct rihvr_ctx {
     ProxForm forced_form = ProxForm::rows;
     // as RIHVR_TEST_BACKTRACKS for RIHVR_TEST_LATE_SCALARS: in those iterations the host finds the block published before
     uint64_t test_late = 0;
-    double test_prev[16] = {};
+    double test_prev[17] = {};
     Timer tm;
     SolveState ss;
 };
@@ -324,6 +325,7 @@ rihvr_status resolve_timing(rihvr_ctx* c) {
 }
 
 static_assert(SL_COUNT == 16 && SL_SEQ == SL_COUNT - 1, "the context's blocks of scalars");
+constexpr int kBlock = SL_COUNT + 1;
 
 // A block of scalars as the host works with it.  The residual norms are reduced over spectra
 // FFT(r) / N: |r|^2 = N sum |FFT(r) / N|^2.
@@ -335,10 +337,24 @@ void take_scalars(rihvr_ctx* c, const double* block) {
 
 // A block of scalars from the device, in stream order
 rihvr_status copy_scalars(rihvr_ctx* c, const double* from) {
-    RIHVR_HIP(hipMemcpyAsync(c->h_scal + SL_COUNT, from, SL_COUNT * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    RIHVR_HIP(hipMemcpyAsync(c->h_scal + kBlock, from, SL_COUNT * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     RIHVR_HIP(hipStreamSynchronize(c->stream));
-    take_scalars(c, c->h_scal + SL_COUNT);
+    take_scalars(c, c->h_scal + kBlock);
     return RIHVR_OK;
+}
+
+// Whether the published block is whole and number `seq`; its values as they were when checked
+bool published_block(const volatile double* host, double seq, double (&block)[SL_COUNT]) {
+    uint64_t sum = 0, check;
+    for (int i = 0; i < SL_COUNT; ++i) {
+        block[i] = host[i];
+        uint64_t bits;
+        std::memcpy(&bits, &block[i], sizeof(bits));
+        sum += check_word(bits, i);
+    }
+    const double word = host[SL_COUNT];
+    std::memcpy(&check, &word, sizeof(check));
+    return sum == check && block[SL_SEQ] == seq;
 }
 
 rihvr_status fetch_scalars(rihvr_ctx* c) {
@@ -349,20 +365,21 @@ rihvr_status fetch_scalars(rihvr_ctx* c) {
 // The scalars as A's reduction (forward_finish) published them, waited for by an event recorded after
 // it, so that work queued later keeps the device busy.  The host decides the solve's path from them
 // (backtracks, the step, restarts) while the device goes by its own copy, so a block of another
-// iteration would not show as an error but as a wrong volume: the block's number is compared, and one
-// that is late is counted and taken by a copy after everything queued.
+// iteration, or half of one, would not show as an error but as a wrong volume: its number and check word
+// are compared, and one that is late is counted and taken by a copy after everything queued.
 rihvr_status wait_scalars(rihvr_ctx* c) {
     RIHVR_HIP(hipEventSynchronize(c->ev_scal));
     if (c->test_late && c->ss.iters < 64) {
-        double now[SL_COUNT];
+        double now[kBlock];
         std::memcpy(now, c->h_scal, sizeof(now));
-        if ((c->test_late >> c->ss.iters) & 1ull) std::memcpy(c->h_scal, c->test_prev, sizeof(now));
+        // (in odd iterations only the block's first half)
+        if ((c->test_late >> c->ss.iters) & 1ull)
+            std::memcpy(c->h_scal, c->test_prev, (c->ss.iters & 1 ? SL_COUNT / 2 : kBlock) * sizeof(double));
         std::memcpy(c->test_prev, now, sizeof(now));
     }
-    double seq;
-    __atomic_load(c->h_scal + SL_SEQ, &seq, __ATOMIC_ACQUIRE);
-    if (seq == c->published) {
-        take_scalars(c, c->h_scal);
+    double block[SL_COUNT];
+    if (published_block(c->h_scal, c->published, block)) {
+        take_scalars(c, block);
     } else {
         ++c->counters.late_scalars;
         RIHVR_TRY(copy_scalars(c, c->scal_pub));
@@ -824,7 +841,7 @@ rihvr_status create_impl(const rihvr_params* params, const rihvr_schedule* sch, 
     RIHVR_TRY(dalloc(&c->dflag, 4));
     RIHVR_TRY(dalloc(&c->d_smom, 1));
     RIHVR_TRY(dalloc(&c->d_step, 1));
-    RIHVR_HIP(hipHostMalloc((void**)&c->h_scal, 2 * SL_COUNT * sizeof(double), hipHostMallocDefault));
+    RIHVR_HIP(hipHostMalloc((void**)&c->h_scal, (kBlock + SL_COUNT) * sizeof(double), hipHostMallocDefault));
 
     // kappa table, plane list and per-plane phase factors, computed on the host
     // exactly as the reference does (sparse_compressive_holo.cu:38-56;

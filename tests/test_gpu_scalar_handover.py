@@ -1,6 +1,7 @@
-"""The scalars of an iteration reach the host with a number, and a block that is not the iteration's is
-not used: with RIHVR_TEST_LATE_SCALARS the host finds the block published before in the given iterations
-(of the first iteration too, where that is the solve before's or none), and the solve must come out
+"""The scalars of an iteration reach the host with a number and a check word, and a block that is not the
+iteration's, or not whole, is not used: with RIHVR_TEST_LATE_SCALARS the host finds the block published
+before in the given iterations (of the first iteration too, where that is the solve before's or none; in
+odd iterations only the first half of that block), and the solve must come out
 the same bit for bit, volume, objectives and decisions, with every late block counted.  Without it
 none is late.  With graphs and without, in the modes that hand scalars over, and with backtracks in
 the same iterations."""
