@@ -16,6 +16,8 @@
  * Pointers are plain addresses.  Each data argument carries a location flag
  * (RIHVR_HOST or RIHVR_DEVICE); device pointers must live on the context's GPU.
  * Calls are blocking: when a call returns, its outputs are complete.
+ * Device inputs must be complete, and device outputs free of pending work, when a call
+ * is made: the context's streams do not wait for the caller's.
  * No entry point throws; every one returns an rihvr_status.
  * One context per host thread; a context owns its device memory, its HIP stream
  * and its FFT schedules.  Contexts share no state.

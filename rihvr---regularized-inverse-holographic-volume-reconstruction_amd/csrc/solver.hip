@@ -1015,6 +1015,11 @@ uint64_t weight_bits(const rihvr_ctx* c) {
     return ((uint64_t)a << 32) | b;
 }
 
+// Graphs that a context holds for each half of an iteration.  Solves with one set of weights meet up to
+// about 160 in all (the ring's and maps' rotations, the prox's forms, a few steps); other weights and
+// steps add theirs, and beyond this number the oldest are dropped.
+constexpr size_t kMaxGraphs = 256;
+
 // Replays the graph cached for (key, t) on the context's stream, or captures `enqueue`'s launches
 // into one first.  `bookkeep` performs the host-side state changes of the launches (it runs after
 // a replay; a capture runs `enqueue`, which performs them itself).
@@ -1039,7 +1044,13 @@ rihvr_status graph_run(rihvr_ctx* c, int which, const std::vector<const void*>& 
     const hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
     (void)hipGraphDestroy(graph);
     RIHVR_HIP(ie);
-    c->gcache[which].push_back({key, t, exec});
+    std::vector<rihvr_ctx::CachedGraph>& held = c->gcache[which];
+    if (held.size() >= kMaxGraphs) {
+        (void)hipStreamSynchronize(c->stream);  // a replay of it may be in flight
+        (void)hipGraphExecDestroy(held.front().exec);
+        held.erase(held.begin());
+    }
+    held.push_back({key, t, exec});
     RIHVR_HIP(hipGraphLaunch(exec, c->stream));
     return RIHVR_OK;
 }
