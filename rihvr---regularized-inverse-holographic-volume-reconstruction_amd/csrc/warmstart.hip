@@ -57,9 +57,11 @@ __device__ __forceinline__ unsigned short f2bf(float f) {
 // The products of two taps in one MFMA (K = 32): lane group q holds channels 8 (q & 1) .. + 7 of the
 // first tap (q < 2) or the second in 16 bytes, of voxel r16 in a and of output channel r16 in b.
 // Half the matrix instructions and LDS reads of one tap at K = 16, and 16 lanes read 256 contiguous
-// bytes instead of every other 8.  A single tap left over runs with zeros in the second's place: a
-// K = 16 MFMA right after a K = 32 one on the same accumulator gave results that differed from run to
-// run.  One tap at a time, then two: prediction at 128 x 1024^2 19.8 -> 18.0 ms (the 16-channel layers
+// bytes instead of every other 8.  A single tap left over runs with zeros in the second's place.  As a
+// K = 16 MFMA after the K = 32 ones, on the same accumulator, it gave results that differed from run to
+// run in the parity form of k_conv_dma (and nowhere else): the form also has its LDS copies in flight,
+// and this file is built with -amdgpu-mfma-vgpr-form.  Its waits and barriers read right and the cause
+// was not found; here no accumulator chain mixes the two, and the results repeat.  One tap at a time, then two: prediction at 128 x 1024^2 19.8 -> 18.0 ms (the 16-channel layers
 // 8.0 -> 7.8 and 3.63 -> 3.46, now held by the staging, the others 5.3 -> 3.9), loss and gradient at
 // 64 x 128^2 1.96 -> 1.71 ms.
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
