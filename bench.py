@@ -696,7 +696,9 @@ def main():
             "valu_issue_frac": valu_issue,
             "note": ("FP32 operations counted per voxel (prox_flops_per_voxel) against the published FP32 vector "
                      "peak, which assumes packed dual-issue FP32; this build compiles without packed FP32, so "
-                     "its issue ceiling is half of it; valu_issue_frac is the measured fraction of that ceiling"
+                     "its issue ceiling is half of it; valu_issue_frac is the measured fraction of that ceiling; "
+                     "the count is for every voxel, also of rows that the scan for zero rows leaves out (there "
+                     "the kernel reads the gradient: hbm_achieved_GBps)"
                      if bound == "valu" else None),
             "line_fraction": f_line,
         },
